@@ -381,6 +381,16 @@ int sdf_nn(const float *points, const float *aabb_tree, const float *queries,
            uint32_t num_points, uint32_t num_queries, uint32_t *indices,
            void *stream);
 
+/* sdf_nn with scratch, for the same results sooner: few points times queries
+ * are scanned, else points and queries are sorted along a curve for the call
+ * (a stream in capture searches the tree as sdf_nn does).  scratch:
+ * sdf_nn_scratch_bytes(num_points, num_queries), 256-byte aligned. */
+size_t sdf_nn_scratch_bytes(uint32_t num_points, uint32_t num_queries);
+int sdf_nn_planned(const float *points, const float *aabb_tree,
+                   const float *queries, uint32_t num_points,
+                   uint32_t num_queries, uint32_t *indices, void *scratch,
+                   size_t scratch_bytes, void *stream);
+
 /* Start cell of each ray: the nearest point to its origin (rays [num_rays, 6],
  * origin first), as sdf_nn over the distinct origins gives it for finite
  * points and origins (ties: smallest index), without a host synchronisation:

@@ -63,6 +63,8 @@ EXPORTS = (
     "sdf_delaunay_certify_points",
     "sdf_delaunay_merge_verified",
     "sdf_nn",
+    "sdf_nn_scratch_bytes",
+    "sdf_nn_planned",
     "sdf_trace_walk_stats",
     "sdf_debug_fpmath",
     "sdf_set_timing",
@@ -242,6 +244,10 @@ def lib() -> C.CDLL:
                                               C.c_uint64, P, P, C.c_uint64, P, P, SZ, P]
     L.sdf_nn.restype = C.c_int
     L.sdf_nn.argtypes = [P, P, P, U32, U32, P, P]
+    L.sdf_nn_scratch_bytes.restype = SZ
+    L.sdf_nn_scratch_bytes.argtypes = [U32, U32]
+    L.sdf_nn_planned.restype = C.c_int
+    L.sdf_nn_planned.argtypes = [P, P, P, U32, U32, P, P, SZ, P]
     L.sdf_trace_walk_stats.restype = C.c_int
     L.sdf_trace_walk_stats.argtypes = [
         C.c_int, C.POINTER(TraceSettings), C.c_int, U32, P, P, U32, P, P, U32, P, P, P,

@@ -31,63 +31,125 @@ __device__ __host__ inline uint32_t pow2_up(uint32_t x) {
     return r;
 }
 
-// leaves (src/aabb_tree/aabb_tree.cu:192-221)
-__global__ __launch_bounds__(kBlock) void build_leaves_kernel(const float *__restrict__ points,
-                                                              uint32_t num_points, uint32_t leaves,
-                                                              float *__restrict__ tree) {
-    const uint32_t l = blockIdx.x * kBlock + threadIdx.x;
-    if (l == 0) {
-        // the unused last entry of the [pow2(N), 2, 3] array
-        float *z = tree + 6ull * (2ull * leaves - 1);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) z[c] = 0.0f;
-    }
-    if (l >= leaves) return;
-    const uint32_t pi = 2 * l;
-    const float *a = points + 3ull * (pi < num_points ? pi : num_points - 1);
-    const float *b = (pi + 1 < num_points) ? points + 3ull * (pi + 1) : a;
-    float *node = tree + 6ull * l;
+struct Box {
+    float v[6]; // min x, y, z, max x, y, z
+};
+
+__device__ __forceinline__ Box join(const Box &a, const Box &b) {
+    Box r;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        const float av = a[c], bv = b[c];
-        node[c] = fminf(av, bv);
-        node[3 + c] = fmaxf(av, bv);
+        r.v[c] = fminf(a.v[c], b.v[c]);
+        r.v[3 + c] = fmaxf(a.v[3 + c], b.v[3 + c]);
     }
+    return r;
 }
 
-// one level above `child_start` (src/aabb_tree/aabb_tree.cu:254-292)
-__global__ __launch_bounds__(kBlock) void build_level_kernel(float *__restrict__ tree,
-                                                             uint64_t child_start, uint32_t width) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= width) return;
-    const float *c0 = tree + 6ull * (child_start + 2ull * i);
-    const float *c1 = c0 + 6;
-    float *node = tree + 6ull * (child_start + 2ull * width + i);
+__device__ __forceinline__ void store_box(float *__restrict__ tree, uint64_t node, const Box &b) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        node[c] = fminf(c0[c], c1[c]);
-        node[3 + c] = fmaxf(c0[c + 3], c1[c + 3]);
+    for (int c = 0; c < 6; ++c) tree[6ull * node + c] = b.v[c];
+}
+
+// Eleven tree levels per launch.  A block takes kBuildNodes consecutive nodes
+// of the level that starts at node `start` and is `width` nodes wide (a power
+// of two): with LEAVES it makes them from point pairs (src/aabb_tree/
+// aabb_tree.cu:192-221), else it reads them; each thread joins four of them in
+// registers and the block's 256 results go up eight more levels through LDS
+// (src/aabb_tree/aabb_tree.cu:254-292, the same pairs).  One launch per level,
+// before, was bound by the launches: 20 of them at 1M points, 55 us of GPU
+// time and ~100 us of host time, against two launches and 19.5 us.
+constexpr uint32_t kBuildNodes = 4 * kBlock;
+
+template <bool LEAVES>
+__global__ __launch_bounds__(kBlock) void build_levels_kernel(const float *__restrict__ points,
+                                                              uint32_t num_points,
+                                                              float *__restrict__ tree,
+                                                              uint64_t start, uint32_t width) {
+    __shared__ float up[6][kBlock];
+    const uint32_t t = threadIdx.x;
+    const uint64_t first = (uint64_t)blockIdx.x * kBuildNodes + 4u * t; // of the level
+    if (LEAVES && blockIdx.x == 0 && t == 0) {
+        // the unused last entry of the [pow2(N), 2, 3] array
+        const Box zero = {{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}};
+        store_box(tree, 2ull * width - 1, zero);
+    }
+    Box n[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint64_t i = first + k;
+        if (i >= width) break;
+        if constexpr (LEAVES) {
+            // the last point repeated as padding
+            const uint64_t p = 2ull * i;
+            const float *a = points + 3ull * (p < num_points ? p : num_points - 1u);
+            const float *b = p + 1 < num_points ? points + 3ull * (p + 1) : a;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                n[k].v[c] = fminf(a[c], b[c]);
+                n[k].v[3 + c] = fmaxf(a[c], b[c]);
+            }
+            store_box(tree, i, n[k]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) n[k].v[c] = tree[6ull * (start + i) + c];
+        }
+    }
+    // two levels in registers (a level of width w has w / 2 parents)
+    uint64_t at = start + width;
+    uint32_t w = width / 2;
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        n[k] = join(n[2 * k], n[2 * k + 1]);
+        if (first / 2 + k < w) store_box(tree, at + first / 2 + k, n[k]);
+    }
+    at += w;
+    w /= 2;
+    n[0] = join(n[0], n[1]);
+    if (first / 4 < w) store_box(tree, at + first / 4, n[0]);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) up[c][t] = n[0].v[c];
+    // eight more through LDS: thread t < live joins entries 2 t, 2 t + 1
+    for (uint32_t live = kBlock / 2; live >= 1; live /= 2) {
+        at += w;
+        w /= 2;
+        if (w == 0) break; // the whole grid: the root is done
+        __syncthreads();
+        Box r;
+        if (t < live) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                r.v[c] = fminf(up[c][2 * t], up[c][2 * t + 1]);
+                r.v[3 + c] = fmaxf(up[3 + c][2 * t], up[3 + c][2 * t + 1]);
+            }
+            const uint64_t i = (uint64_t)blockIdx.x * live + t;
+            if (i < w) store_box(tree, at + i, r);
+        }
+        __syncthreads();
+        if (t < live) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) up[c][t] = r.v[c];
+        }
     }
 }
 
 hipError_t launch_build_aabb_tree(const float *points, uint32_t num_points, float *tree,
                                   hipStream_t stream) {
-    const uint32_t n2 = pow2_up(num_points);
-    const uint32_t leaves = n2 / 2;
-    if (leaves == 0) return hipSuccess;
-    hipLaunchKernelGGL(build_leaves_kernel, dim3((leaves + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                       stream, points, num_points, leaves, tree);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    uint32_t width = pow2_up(num_points) / 2;
+    if (width == 0) return hipSuccess;
+    auto grid = [](uint32_t w) { return dim3((w + kBuildNodes - 1) / kBuildNodes); };
+    hipLaunchKernelGGL(build_levels_kernel<true>, grid(width), dim3(kBlock), 0, stream, points,
+                       num_points, tree, 0ull, width);
     uint64_t start = 0;
-    for (uint32_t width = leaves / 2; width >= 1; width /= 2) {
-        hipLaunchKernelGGL(build_level_kernel, dim3((width + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                           stream, tree, start, width);
-        e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        start += 2ull * width;
+    while (width > kBuildNodes) {
+        // the launch before ended with one node per block
+        for (uint32_t k = kBuildNodes; k > 1; k /= 2) {
+            start += width;
+            width /= 2;
+        }
+        hipLaunchKernelGGL(build_levels_kernel<false>, grid(width), dim3(kBlock), 0, stream,
+                           points, num_points, tree, start, width);
     }
-    return hipSuccess;
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -317,27 +379,36 @@ __global__ __launch_bounds__(kBlock) void start_init_kernel(uint32_t *__restrict
 // Each ray claims the first free slot of its probe sequence or finds the
 // slot of an equal origin there.  The table has at least twice as many slots
 // as rays, so every probe sequence reaches a free slot or its origin's.
-// Rays of one wavefront with the bits of its first ray's origin take that
-// ray's slot without probing: a batch from one camera then makes one probe
-// per wavefront instead of every ray contending for the same slot.
-__global__ __launch_bounds__(kBlock) void start_hash_kernel(const float *__restrict__ rays,
-                                                            uint32_t num_rays,
-                                                            uint32_t *__restrict__ table,
-                                                            uint64_t slots,
-                                                            uint32_t *__restrict__ ray_slot) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= num_rays) return;
-    const uint32_t *o = reinterpret_cast<const uint32_t *>(rays + 6ull * i);
-    const uint32_t ox = o[0], oy = o[1], oz = o[2];
-    // the first active lane's id and origin, read by every lane (before any
-    // branch: a cross-lane read in a branch sees only the lanes in it)
-    const uint32_t lead = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & 63u));
-    const uint32_t lx = (uint32_t)__builtin_amdgcn_readfirstlane((int)ox);
-    const uint32_t ly = (uint32_t)__builtin_amdgcn_readfirstlane((int)oy);
-    const uint32_t lz = (uint32_t)__builtin_amdgcn_readfirstlane((int)oz);
-    const bool follower = ((threadIdx.x & 63u) != lead) & (ox == lx) & (oy == ly) & (oz == lz);
+// Rays of one block with the bits of its first ray's origin take that ray's
+// slot without probing: a batch from one camera makes one probe per 1,024 rays
+// instead of every ray contending for the same slot.  (One probe per wavefront,
+// before, left 30,000 of them for one line of the table at 1600x1200 rays: 110 us
+// against 19 us now.)
+constexpr uint32_t kHashBlock = 1024;
+
+__global__ __launch_bounds__(kHashBlock) void start_hash_kernel(const float *__restrict__ rays,
+                                                                uint32_t num_rays,
+                                                                uint32_t *__restrict__ table,
+                                                                uint64_t slots,
+                                                                uint32_t *__restrict__ ray_slot) {
+    __shared__ uint32_t lead[4]; // the first ray's origin and slot
+    const uint32_t i = blockIdx.x * kHashBlock + threadIdx.x;
+    uint32_t ox = 0, oy = 0, oz = 0;
+    if (i < num_rays) {
+        const uint32_t *o = reinterpret_cast<const uint32_t *>(rays + 6ull * i);
+        ox = o[0];
+        oy = o[1];
+        oz = o[2];
+    }
+    if (threadIdx.x == 0) {
+        lead[0] = ox;
+        lead[1] = oy;
+        lead[2] = oz;
+    }
+    __syncthreads();
+    const bool follower = threadIdx.x != 0 && ox == lead[0] && oy == lead[1] && oz == lead[2];
     uint64_t h = origin_hash(ox, oy, oz) & (slots - 1);
-    if (!follower) {
+    if (i < num_rays && !follower) {
         for (uint64_t probe = 0; probe < slots; ++probe) {
             uint32_t s = table[h];
             if (s == kNoIndex) {
@@ -348,9 +419,9 @@ __global__ __launch_bounds__(kBlock) void start_hash_kernel(const float *__restr
             h = (h + 1) & (slots - 1);
         }
     }
-    // the first ray's slot (its probe has ended: the loop above is done)
-    const uint32_t lead_slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)h);
-    ray_slot[i] = follower ? lead_slot : (uint32_t)h;
+    if (threadIdx.x == 0) lead[3] = (uint32_t)h;
+    __syncthreads();
+    if (i < num_rays) ray_slot[i] = follower ? lead[3] : (uint32_t)h;
 }
 
 // Numbers the claimed slots (the distinct origins) and resets their results.
@@ -371,9 +442,63 @@ __global__ __launch_bounds__(kBlock) void start_unique_kernel(const uint32_t *__
     }
 }
 
+// Nearest of the block's kBlock * kStartPts points (block `chunk` of them) to
+// each of the `count` positions q: per position one atomic of the smallest
+// (distance bits, index) into best.  Lanes keep their own smallest over their
+// points; the wave's smallest distance comes by DPP and its index from the
+// lanes that hold that distance (one, but for ties).
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+    auto step = [](uint32_t x, uint32_t y) { return x < y ? x : y; };
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));
+    v = step(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ void brute_scan(const float *__restrict__ points, uint32_t num_points,
+                                           uint32_t chunk, const float (*q)[3], uint32_t count,
+                                           unsigned long long *slot, uint64_t *__restrict__ best) {
+    const uint64_t p0 = (uint64_t)chunk * kBlock * kStartPts + threadIdx.x;
+    float px[kStartPts], py[kStartPts], pz[kStartPts];
+#pragma unroll
+    for (uint32_t k = 0; k < kStartPts; ++k) {
+        const uint64_t j = p0 + (uint64_t)k * kBlock;
+        // past the end: NaN, no candidate
+        const bool ok = j < num_points;
+        px[k] = ok ? points[3 * j] : __builtin_bit_cast(float, 0x7fc00000u);
+        py[k] = ok ? points[3 * j + 1] : 0.0f;
+        pz[k] = ok ? points[3 * j + 2] : 0.0f;
+    }
+    for (uint32_t u = 0; u < count; ++u) {
+        const float qx = q[u][0], qy = q[u][1], qz = q[u][2];
+        uint32_t dist = 0xffffffffu, at = 0u; // distances are >= 0: their bits sort like them
+#pragma unroll
+        for (uint32_t k = 0; k < kStartPts; ++k) {
+            const float dx = px[k] - qx, dy = py[k] - qy, dz = pz[k] - qz;
+            const float d = sqrtf(sdf_dot3(dx, dy, dz, dx, dy, dz));
+            const uint32_t b = __builtin_bit_cast(uint32_t, d);
+            if (d == d && b < dist) { // points in ascending order: ties keep the first
+                dist = b;
+                at = k;
+            }
+        }
+        const uint32_t least = wave_min_u32(dist);
+        if (least == 0xffffffffu) continue; // no point of the wave has a distance
+        const uint32_t j = (uint32_t)(p0 + (uint64_t)at * kBlock);
+        const uint32_t first = wave_min_u32(dist == least ? j : 0xffffffffu);
+        if ((threadIdx.x & 63u) == 0)
+            atomicMin(slot + u, (unsigned long long)least << 32 | first);
+    }
+    __syncthreads();
+    for (uint32_t u = threadIdx.x; u < count; u += kBlock)
+        if (slot[u] != ~0ull) atomicMin(reinterpret_cast<unsigned long long *>(best) + u, slot[u]);
+}
+
 // At most kStartBrute distinct origins: every block scans kBlock * kStartPts
-// points for all of them; per origin the smallest (distance bits, index)
-// of the block goes into `best` with one atomic.
+// points for all of them.
 __global__ __launch_bounds__(kBlock) void start_brute_kernel(const float *__restrict__ points,
                                                              uint32_t num_points,
                                                              const float *__restrict__ rays,
@@ -392,38 +517,57 @@ __global__ __launch_bounds__(kBlock) void start_brute_kernel(const float *__rest
         slot[u] = ~0ull;
     }
     __syncthreads();
-    const uint64_t p0 = (uint64_t)blockIdx.x * kBlock * kStartPts;
-    float px[kStartPts], py[kStartPts], pz[kStartPts];
+    brute_scan(points, num_points, blockIdx.x, q, count, slot, best);
+}
+
+// The same for nn's queries, kScanQueries of them per blockIdx.y (a block takes
+// its queries one after another, 0.7 us each: with 256 of them 1,000 queries
+// over 4,096 points took 192 us on 8 blocks).
+constexpr uint32_t kScanQueries = 64;
+
+__global__ __launch_bounds__(kBlock) void nn_brute_kernel(const float *__restrict__ points,
+                                                          uint32_t num_points,
+                                                          const float *__restrict__ queries,
+                                                          uint32_t num_queries,
+                                                          uint64_t *__restrict__ best) {
+    __shared__ float q[kScanQueries][3];
+    __shared__ unsigned long long slot[kScanQueries];
+    const uint32_t q0 = blockIdx.y * kScanQueries;
+    const uint32_t count = min(kScanQueries, num_queries - q0);
+    if (threadIdx.x < count) {
+        const uint32_t u = threadIdx.x;
 #pragma unroll
-    for (uint32_t k = 0; k < kStartPts; ++k) {
-        const uint64_t j = p0 + (uint64_t)k * kBlock + threadIdx.x;
-        const bool ok = j < num_points;
-        px[k] = ok ? points[3 * j] : 0.0f;
-        py[k] = ok ? points[3 * j + 1] : 0.0f;
-        pz[k] = ok ? points[3 * j + 2] : 0.0f;
-    }
-    for (uint32_t u = 0; u < count; ++u) {
-        const float qx = q[u][0], qy = q[u][1], qz = q[u][2];
-        unsigned long long key = ~0ull;
-#pragma unroll
-        for (uint32_t k = 0; k < kStartPts; ++k) {
-            const uint64_t j = p0 + (uint64_t)k * kBlock + threadIdx.x;
-            const float dx = px[k] - qx, dy = py[k] - qy, dz = pz[k] - qz;
-            const float d = sqrtf(sdf_dot3(dx, dy, dz, dx, dy, dz));
-            const unsigned long long c =
-                ((unsigned long long)__builtin_bit_cast(uint32_t, d) << 32) | (uint32_t)j;
-            if (j < num_points && d == d && c < key) key = c; // NaN: no candidate
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const unsigned long long o = __shfl_xor(key, off, 64);
-            key = o < key ? o : key;
-        }
-        if ((threadIdx.x & 63u) == 0 && key != ~0ull) atomicMin(slot + u, key);
+        for (int c = 0; c < 3; ++c) q[u][c] = queries[3ull * (q0 + u) + c];
+        slot[u] = ~0ull;
     }
     __syncthreads();
-    for (uint32_t u = threadIdx.x; u < count; u += kBlock)
-        if (slot[u] != ~0ull) atomicMin(reinterpret_cast<unsigned long long *>(best) + u, slot[u]);
+    brute_scan(points, num_points, blockIdx.x, q, count, slot, best + q0);
+}
+
+__global__ __launch_bounds__(kBlock) void nn_reset_kernel(uint64_t *__restrict__ best, uint32_t n) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) best[i] = ~0ull;
+}
+
+__global__ __launch_bounds__(kBlock) void nn_result_kernel(const uint64_t *__restrict__ best,
+                                                           uint32_t n,
+                                                           uint32_t *__restrict__ indices) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) indices[i] = best[i] == ~0ull ? 0u : (uint32_t)best[i];
+}
+
+hipError_t launch_nn_brute(const float *points, const float *queries, uint32_t num_points,
+                           uint32_t num_queries, uint32_t *indices, uint64_t *best,
+                           hipStream_t stream) {
+    const dim3 per_query((num_queries + kBlock - 1) / kBlock);
+    const dim3 grid((uint32_t)(((uint64_t)num_points + kBlock * kStartPts - 1) / (kBlock * kStartPts)),
+                    (num_queries + kScanQueries - 1) / kScanQueries);
+    hipLaunchKernelGGL(nn_reset_kernel, per_query, dim3(kBlock), 0, stream, best, num_queries);
+    hipLaunchKernelGGL(nn_brute_kernel, grid, dim3(kBlock), 0, stream, points, num_points, queries,
+                       num_queries, best);
+    hipLaunchKernelGGL(nn_result_kernel, per_query, dim3(kBlock), 0, stream, best, num_queries,
+                       indices);
+    return hipGetLastError();
 }
 
 // More distinct origins: one tree search per origin, the waves of the grid
@@ -475,8 +619,8 @@ hipError_t launch_start_points(const float *rays, uint32_t num_rays, const float
     const uint32_t ray_blocks = (num_rays + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(start_init_kernel, dim3(slot_blocks), dim3(kBlock), 0, stream, counter, table,
                        l.table_slots);
-    hipLaunchKernelGGL(start_hash_kernel, dim3(ray_blocks), dim3(kBlock), 0, stream, rays, num_rays,
-                       table, l.table_slots, ray_slot);
+    hipLaunchKernelGGL(start_hash_kernel, dim3((num_rays + kHashBlock - 1) / kHashBlock),
+                       dim3(kHashBlock), 0, stream, rays, num_rays, table, l.table_slots, ray_slot);
     hipLaunchKernelGGL(start_unique_kernel, dim3(slot_blocks), dim3(kBlock), 0, stream, table,
                        l.table_slots, counter, uid, uq_ray, best);
     const uint32_t point_blocks = (uint32_t)(((uint64_t)num_points + kBlock * kStartPts - 1) /

@@ -926,6 +926,44 @@ int sdf_nn(const float *points, const float *aabb_tree, const float *queries, ui
     return SDF_OK;
 }
 
+size_t sdf_nn_scratch_bytes(uint32_t num_points, uint32_t num_queries) {
+    if (num_points < 32 || num_points > kMaxTreePoints) return 0;
+    return nn_scratch_bytes(num_points, num_queries);
+}
+
+int sdf_nn_planned(const float *points, const float *aabb_tree, const float *queries,
+                   uint32_t num_points, uint32_t num_queries, uint32_t *indices, void *scratch,
+                   size_t scratch_bytes, void *stream) {
+    if (num_points < 32) return fail(SDF_E_INVALID, "number of points must be at least 32");
+    if (num_points > kMaxTreePoints)
+        return fail(SDF_E_INVALID, "at most %u points (got %u)", kMaxTreePoints, num_points);
+    if (!points || !aabb_tree || (num_queries > 0 && (!queries || !indices)))
+        return fail(SDF_E_INVALID, "NULL pointer argument");
+    if (num_queries == 0) return SDF_OK;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    // a captured graph holds no memset nodes, which the sorts would record
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool scans = nn_scans(num_points, num_queries);
+    if (!scans && hipStreamIsCapturing(s, &capture) == hipSuccess &&
+        capture != hipStreamCaptureStatusNone)
+        return sdf_nn(points, aabb_tree, queries, num_points, num_queries, indices, stream);
+    const size_t need = sdf_nn_scratch_bytes(num_points, num_queries);
+    if (need == 0) return fail(SDF_E_HIP, "nn: the sort's scratch could not be sized");
+    if (!scratch || scratch_bytes < need)
+        return fail(SDF_E_INVALID, "scratch must hold %zu bytes (got %zu)", need, scratch_bytes);
+    if ((reinterpret_cast<uintptr_t>(scratch) & 255u) != 0)
+        return fail(SDF_E_INVALID, "scratch must be 256-byte aligned");
+    tbegin(SDF_KERNEL_NN, s);
+    const hipError_t e =
+        scans ? launch_nn_brute(points, queries, num_points, num_queries, indices,
+                                static_cast<uint64_t *>(scratch), s)
+              : launch_nn_sorted(points, aabb_tree, queries, num_points, num_queries, indices,
+                                 scratch, s);
+    tend(s);
+    if (e != hipSuccess) return hip_fail(e, "nn");
+    return SDF_OK;
+}
+
 size_t sdf_start_points_scratch_bytes(uint32_t num_rays) {
     return start_layout(num_rays).bytes;
 }

@@ -52,7 +52,6 @@ def nn(points: torch.Tensor, tree: torch.Tensor, queries: torch.Tensor) -> torch
         raise RuntimeError("tree must be on CUDA device")
     if queries.device.type != "cuda":
         raise RuntimeError("queries must be on CUDA device")
-    indices = torch.zeros(tuple(queries.shape[:-1]), dtype=torch.uint32, device=queries.device)
     if num_points < 32:
         raise RuntimeError("number of points must be at least 32")
     if _scalar_type(points.dtype) != "float32":
@@ -60,9 +59,15 @@ def nn(points: torch.Tensor, tree: torch.Tensor, queries: torch.Tensor) -> torch
     p = points.contiguous()
     t = tree.contiguous()
     q = queries.contiguous()
+    # every query's index is written
+    indices = torch.empty(tuple(queries.shape[:-1]), dtype=torch.uint32, device=queries.device)
+    L = _lib.lib()
     with torch.cuda.device(q.device):
-        check(_lib.lib().sdf_nn(ptr(p), ptr(t), ptr(q), num_points, num_queries, ptr(indices),
-                                _lib.stream_handle(q.device)))
+        nbytes = int(L.sdf_nn_scratch_bytes(num_points, num_queries))
+        scratch = torch.empty(nbytes + 256, dtype=torch.uint8, device=q.device)
+        check(L.sdf_nn_planned(ptr(p), ptr(t), ptr(q), num_points, num_queries, ptr(indices),
+                               (scratch.data_ptr() + 255) & ~255, nbytes,
+                               _lib.stream_handle(q.device)))
     return indices
 
 
