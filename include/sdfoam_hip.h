@@ -271,7 +271,19 @@ typedef struct sdf_trace_plan {
     uint32_t walk_record_chunks; /* chunks of 16 trips in the record's pool, rounded up to
                                     a multiple of 8; 0: every wavefront's `walk_budget`
                                     trips (sdf_walk_record_full_chunks) */
+    uint32_t outputs;          /* SDF_OUTPUTS_* bits, 0: per-point outputs are zeroed by
+                                  the caller and added to */
 } sdf_trace_plan;
+
+/* The per-point outputs hold nothing yet and are written instead of added to.
+ * Forward (needs cell_table): point_contribution and alpha_output.  Backward
+ * (needs grad_accum): attribute_grad, points_grad, point_error and
+ * sharpness_grad[0]. */
+#define SDF_OUTPUTS_FRESH 1u
+/* Backward (with SDF_OUTPUTS_FRESH): non-finite gradients (not the point
+ * error) are written as 0, as TraceRays does to them
+ * (sdfoam_model/render.py:166-170). */
+#define SDF_OUTPUTS_FINITE 2u
 
 /* Bytes of a walk record for every wavefront's `budget` trips (a pool that
  * never runs out), and for a pool of `chunks` chunks (0: the same). */

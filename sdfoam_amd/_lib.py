@@ -128,7 +128,12 @@ class TracePlanDesc(C.Structure):
         ("cell_table", C.c_void_p),
         ("cell_table_bytes", C.c_size_t),
         ("walk_record_chunks", C.c_uint32),
+        ("outputs", C.c_uint32),
     ]
+
+
+SDF_OUTPUTS_FRESH = 1
+SDF_OUTPUTS_FINITE = 2
 
 
 _lib = None

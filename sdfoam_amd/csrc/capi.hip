@@ -183,6 +183,9 @@ int trace_forward_impl(const sdf_trace_plan *plan, int sh_degree,
             return fail(SDF_E_INVALID, "cell table must be 256-byte aligned");
         cells = static_cast<uint32_t *>(plan->cell_table);
     }
+    const bool fresh = plan && (plan->outputs & SDF_OUTPUTS_FRESH) != 0;
+    if (fresh && !cells)
+        return fail(SDF_E_INVALID, "SDF_OUTPUTS_FRESH needs a cell table in the forward");
     hipStream_t s = static_cast<hipStream_t>(stream);
     FwdArgs a = {};
     a.scene = make_scene(num_points, points, attributes, adjacency_size, point_adjacency,
@@ -191,7 +194,9 @@ int trace_forward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (cells) {
         // the offset table and the cell table in one pass
         tbegin(SDF_KERNEL_SCENE_PREP, s);
-        e = launch_scene_prep(sh_degree, half, a.scene, cells, static_cast<uint2 *>(scratch), s);
+        e = launch_scene_prep(sh_degree, half, a.scene, cells, static_cast<uint2 *>(scratch),
+                              fresh ? point_contribution : nullptr,
+                              fresh ? alpha_output : nullptr, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "scene preparation");
         a.scene.cells = cells;
@@ -278,6 +283,11 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
             return fail(SDF_E_INVALID, "gradient accumulator must be 256-byte aligned");
         accum = static_cast<float *>(plan->grad_accum);
     }
+    const uint32_t outputs = plan ? plan->outputs : 0u;
+    if ((outputs & SDF_OUTPUTS_FRESH) != 0 && (!accum || num_rays == 0))
+        return fail(SDF_E_INVALID, "SDF_OUTPUTS_FRESH needs rays and a gradient accumulator in the backward");
+    if (outputs == SDF_OUTPUTS_FINITE)
+        return fail(SDF_E_INVALID, "SDF_OUTPUTS_FINITE needs SDF_OUTPUTS_FRESH");
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
     if (!(plan && plan->scratch_ready)) {
@@ -290,7 +300,8 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (num_rays == 0) return SDF_OK;
     if (accum) {
         tbegin(SDF_KERNEL_GRAD_CLEAR, s);
-        e = launch_grad_clear(sh_degree, accum, num_points, s);
+        e = launch_grad_clear(sh_degree, accum, num_points,
+                              (outputs & SDF_OUTPUTS_FRESH) ? sharpness_grad : nullptr, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "gradient accumulator clear");
     }
@@ -324,7 +335,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (accum) {
         tbegin(SDF_KERNEL_GRAD_FINALIZE, s);
         e = launch_grad_finalize(sh_degree, accum, num_points, attribute_grad, points_grad,
-                                 a.point_error, half, s);
+                                 a.point_error, sharpness_grad, outputs, half, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "gradient accumulator finalize");
     }

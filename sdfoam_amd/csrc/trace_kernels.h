@@ -230,9 +230,10 @@ hipError_t launch_forward(int L, const FwdArgs &a, bool neus, bool stats, bool h
                           hipStream_t stream);
 // Fills the fp16 offset table `diff` (as launch_prefetch_diff) and the cell
 // table (cell_record_bytes(L, attribute size) per cell) from sc's points,
-// adjacency, offsets and attributes, in one pass.
+// adjacency, offsets and attributes, in one pass, and zeroes contribution
+// (attribute type) and alpha [N] where they are given.
 hipError_t launch_scene_prep(int L, bool half, const SceneView &sc, uint32_t *cells, uint2 *diff,
-                             hipStream_t stream);
+                             void *contribution, float *alpha, hipStream_t stream);
 // Floats per cell row of the backward's gradient accumulator: the next
 // power of two >= D + 4 (attribute row, position, point error), at least 8,
 // so that a row spans the fewest 64-byte segments.
@@ -240,15 +241,18 @@ constexpr uint32_t accum_stride(int L) {
     return L <= 0 ? 8u : L <= 2 ? 32u : 64u;
 }
 
-// Clears num_points rows of the accumulator.
-hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, hipStream_t stream);
+// Clears num_points rows of the accumulator, and sharpness_grad[0] if given.
+hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, float *sharpness_grad,
+                             hipStream_t stream);
 
 // attribute_grad [N, D] += rows[:, :D]; points_grad [N, 3] += rows[:, D:D+3];
 // point_error [N] += rows[:, D+3] (point_error may be nullptr).  attr_grad and
 // point_error are fp16 when `half` (the sum is rounded once), else fp32.
+// outputs: SDF_OUTPUTS_* bits; with SDF_OUTPUTS_FINITE sharpness_grad[0] too
+// becomes 0 where it is not finite.
 hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, void *attr_grad,
-                                float *points_grad, void *point_error, bool half,
-                                hipStream_t stream);
+                                float *points_grad, void *point_error, float *sharpness_grad,
+                                uint32_t outputs, bool half, hipStream_t stream);
 
 hipError_t launch_backward(int L, const BwdArgs &a, bool neus, bool stats, bool half,
                            hipStream_t stream);

@@ -203,11 +203,16 @@ class TracePlan:
         self.budget = budget
         self.chunks = chunks
 
+    def record_head(self) -> torch.Tensor:
+        """The record's first bytes (int32 [8 * 64], on the device): a counter
+        every 256 bytes."""
+        off = self.record_ptr - self.entries.data_ptr()
+        return self.entries[off:off + 256 * RECORD_COUNTERS].view(torch.int32)
+
     def record_counters(self) -> torch.Tensor:
         """The record's chunk counters (int32 [8], on the device): their sum
         is the number of chunks the last forward asked for."""
-        off = self.record_ptr - self.entries.data_ptr()
-        return self.entries[off:off + 256 * RECORD_COUNTERS].view(torch.int32)[::64]
+        return self.record_head()[::64]
 
     def desc(self, record_key=None):
         """The C descriptor; the walk record is left out when `record_key`
@@ -239,12 +244,12 @@ class _RecordNeed:
     forward and read once that copy has completed (no synchronisation)."""
 
     def __init__(self):
-        self.host = torch.zeros(RECORD_COUNTERS, dtype=torch.int32).pin_memory()
+        self.host = torch.zeros(64 * RECORD_COUNTERS, dtype=torch.int32, pin_memory=True)
         self.event = None
         self.per_xcd = 0  # the most chunks one XCD asked for
 
     def observe(self, plan: "TracePlan") -> None:
-        self.host.copy_(plan.record_counters(), non_blocking=True)
+        self.host.copy_(plan.record_head(), non_blocking=True)
         self.event = torch.cuda.Event()
         self.event.record()
 
@@ -253,7 +258,7 @@ class _RecordNeed:
         claims from its own eighth of the pool, so the eighths are sized for
         the XCD that asked for most."""
         if self.event is not None and self.event.query():
-            self.per_xcd = int(self.host.max())
+            self.per_xcd = int(self.host[::64].max())
             self.event = None
         if self.per_xcd <= 0:
             return 0
@@ -382,16 +387,18 @@ class Pipeline:
             _lib.SDF_ATTR_F16 if self._attr_dtype == torch.float16 else _lib.SDF_ATTR_F32,
         )
 
-    def _zeros_attr(self, shape, device) -> torch.Tensor:
-        """Zeroed buffer of the attribute type for atomic accumulation: fp16
-        atomics are packed 4-byte words, so an odd element count gets one
-        padding half (the result is a view of the first elements)."""
+    def _attr_buffer(self, shape, device, zero: bool = True) -> torch.Tensor:
+        """Buffer of the attribute type for atomic accumulation, zeroed unless
+        the kernels write it whole: fp16 atomics are packed 4-byte words, so an
+        odd element count gets one padding half (the result is a view of the
+        first elements)."""
+        make = torch.zeros if zero else torch.empty
         n = 1
         for d in shape:
             n *= int(d)
         if self._attr_dtype == torch.float16 and n % 2 == 1:
-            return torch.zeros(n + 1, dtype=self._attr_dtype, device=device)[:n].view(shape)
-        return torch.zeros(shape, dtype=self._attr_dtype, device=device)
+            return make(n + 1, dtype=self._attr_dtype, device=device)[:n].view(shape)
+        return make(shape, dtype=self._attr_dtype, device=device)
 
     @staticmethod
     def _scratch(num_points: int, num_adj: int, device) -> tuple[torch.Tensor, int]:
@@ -465,12 +472,17 @@ class Pipeline:
         lead = tuple(rays_c.shape[:-1])
         rgba = torch.empty(lead + (4,), dtype=self._attr_dtype, device=dev)
         nisect = torch.empty(lead + (1,), dtype=torch.uint32, device=dev)
-        contribution = self._zeros_attr((num_points, 1), dev) if return_contribution else None
-        depth = didx = None
+        # with a cell table the kernels zero the per-point outputs themselves;
+        # every ray writes its own outputs
+        fresh = bool(cell_table) and num_rays > 0
+        contribution = depth = didx = None
+        if return_contribution:
+            contribution = self._attr_buffer((num_points, 1), dev, zero=not fresh)
         if return_depth:
-            depth = torch.zeros(lead + (num_q,), dtype=torch.float32, device=dev)
-            didx = torch.zeros(lead + (num_q,), dtype=torch.uint32, device=dev)
-        alpha = torch.zeros((num_points, 1), dtype=torch.float32, device=dev)
+            depth = torch.empty(lead + (num_q,), dtype=torch.float32, device=dev)
+            didx = torch.empty(lead + (num_q,), dtype=torch.uint32, device=dev)
+        alpha = (torch.empty if fresh else torch.zeros)((num_points, 1), dtype=torch.float32,
+                                                        device=dev)
         scratch, nbytes = self._scratch(num_points, num_adj, dev)
         plan = None
         if record_walk is None:
@@ -510,6 +522,7 @@ class Pipeline:
                 desc = _lib.TracePlanDesc()
             desc.cell_table = (cells.data_ptr() + 255) & ~255
             desc.cell_table_bytes = cbytes
+            desc.outputs = _lib.SDF_OUTPUTS_FRESH
         with torch.cuda.device(dev):
             if desc is None:
                 check(_lib.lib().sdf_trace_forward(*args))
@@ -548,6 +561,19 @@ class Pipeline:
         row of a temporary buffer (256 bytes per cell at SH degree 3) before
         adding them to the outputs (fp16 outputs: rounded once); False
         updates the outputs directly."""
+        return self._backward(points, attributes, point_adjacency, point_adjacency_offsets, rays,
+                              start_point, rgb_out, grad_in, depth_quantiles, depth_indices,
+                              depth_grad_in, ray_error, weight_threshold, max_intersections,
+                              alpha_mode, inv_s, sdf_channel, trace_plan, sort_rays, grad_accum)
+
+    def _backward(self, points, attributes, point_adjacency, point_adjacency_offsets, rays,
+                  start_point, rgb_out, grad_in, depth_quantiles, depth_indices, depth_grad_in,
+                  ray_error, weight_threshold=None, max_intersections=None, alpha_mode=None,
+                  inv_s=None, sdf_channel=None, trace_plan=None, sort_rays=None, grad_accum=True,
+                  autograd=False):
+        """trace_backward; with `autograd` (TraceRays) non-finite gradients
+        come back as 0, written so by the pass that writes them, and without
+        the zeros of "ray_grad"."""
         points_c = points.contiguous()
         attributes_c = attributes.contiguous()
         adj_c = point_adjacency.contiguous()
@@ -613,6 +639,8 @@ class Pipeline:
         rerr = None
         point_error = None
         dev = rays_c.device
+        # through the accumulator every gradient is written, not added to
+        fresh = bool(grad_accum) and num_rays > 0
         if return_error:
             rerr = ray_error.contiguous()
             if rerr.dtype != self._attr_dtype:
@@ -623,7 +651,7 @@ class Pipeline:
                 raise RuntimeError("ray_error must be on CUDA device")
             if rerr.numel() != num_rays:
                 raise RuntimeError("ray_error must have the same batch size as rays")
-            point_error = self._zeros_attr((num_points, 1), dev)
+            point_error = self._attr_buffer((num_points, 1), dev, zero=not fresh)
 
         settings = self._settings(weight_threshold, max_intersections, alpha_mode, sdf_channel, rays_c)
         rgba = rgb_out.contiguous()
@@ -631,10 +659,12 @@ class Pipeline:
             raise RuntimeError("rgb_out must be the forward's rgba output")
 
         num_attr = attributes_c.size(0)
-        attr_grad = self._zeros_attr((num_attr, self.attribute_dim()), dev)
-        points_grad = torch.zeros((num_points, 3), dtype=rays_c.dtype, device=dev)
-        ray_grad = torch.zeros_like(rays_c)
-        sharpness_grad = torch.zeros_like(sharpness, dtype=torch.float32)
+        make = torch.empty if fresh else torch.zeros
+        attr_grad = self._attr_buffer((num_attr, self.attribute_dim()), dev, zero=not fresh)
+        points_grad = make((num_points, 3), dtype=rays_c.dtype, device=dev)
+        # the kernels write the first element of the sharpness' gradient
+        sharpness_grad = (make if sharpness.numel() == 1 else torch.zeros)(
+            sharpness.shape, dtype=torch.float32, device=dev)
         table_ready = False
         # the plan of the forward that produced rgb_out, used by one backward
         # (detached here, so the record does not outlive it with the tensor)
@@ -672,6 +702,7 @@ class Pipeline:
             accum = torch.empty(accum_bytes + 256, dtype=torch.uint8, device=dev)
             desc.grad_accum = (accum.data_ptr() + 255) & ~255
             desc.grad_accum_bytes = accum_bytes
+            desc.outputs = _lib.SDF_OUTPUTS_FRESH | (_lib.SDF_OUTPUTS_FINITE if autograd else 0)
         with torch.cuda.device(dev):
             if trace_plan is None and accum is None:
                 check(_lib.lib().sdf_trace_backward(*args))
@@ -682,9 +713,13 @@ class Pipeline:
         out = {
             "points_grad": points_grad,
             "attr_grad": attr_grad,
-            "ray_grad": ray_grad,
             "sharpness_grad": sharpness_grad,
         }
+        if not autograd:
+            out["ray_grad"] = torch.zeros_like(rays_c)
+        elif not fresh:
+            for g in (points_grad, attr_grad, sharpness_grad):
+                g[~g.isfinite()] = 0
         if return_error:
             out["point_error"] = point_error
         return out

@@ -17,6 +17,8 @@ from __future__ import annotations
 
 import torch
 
+from .pipeline import Pipeline
+
 
 class ErrorBox:
     """Carrier for per-ray error in and per-point error out
@@ -32,6 +34,8 @@ class TraceRays(torch.autograd.Function):
     def forward(ctx, pipeline, _points, _attributes, _point_adjacency, _point_adjacency_offsets,
                 rays, start_point, depth_quantiles, return_contribution, use_sdfoam=False,
                 inv_s=50.0, eps=1e-6, sdf_channel=None):
+        # outputs that no gradient reaches get None, not a buffer of zeros
+        ctx.set_materialize_grads(False)
         ctx.rays = rays
         ctx.start_point = start_point
         ctx.pipeline = pipeline
@@ -73,24 +77,34 @@ class TraceRays(torch.autograd.Function):
     def backward(ctx, grad_rgba, grad_depth, grad_contribution, grad_num_intersections,
                  errbox_grad, grad_alpha):
         del grad_contribution, grad_num_intersections, errbox_grad, grad_alpha
-        results = ctx.pipeline.trace_backward(
-            ctx.points, ctx.attributes, ctx.point_adjacency, ctx.point_adjacency_offsets,
-            ctx.rays, ctx.start_point, ctx.rgba, grad_rgba,
-            ctx.depth_quantiles, ctx.depth_indices, grad_depth, ctx.errbox.ray_error,
-            alpha_mode="sdfoam" if ctx.use_sdfoam else "standard",
-            inv_s=ctx.inv_s,
-            eps=ctx.eps,
-            sdf_channel=ctx.sdf_channel,
-        )
+        if grad_rgba is None:
+            grad_rgba = torch.zeros_like(ctx.rgba)
+        if grad_depth is None and ctx.depth_quantiles is not None:
+            grad_depth = torch.zeros(ctx.depth_quantiles.shape, dtype=torch.float32,
+                                     device=ctx.rgba.device)
+        args = (ctx.points, ctx.attributes, ctx.point_adjacency, ctx.point_adjacency_offsets,
+                ctx.rays, ctx.start_point, ctx.rgba, grad_rgba,
+                ctx.depth_quantiles, ctx.depth_indices, grad_depth, ctx.errbox.ray_error)
+        options = dict(alpha_mode="sdfoam" if ctx.use_sdfoam else "standard", inv_s=ctx.inv_s,
+                       sdf_channel=ctx.sdf_channel)
+        # this package's pipeline zeroes the non-finite gradients as it writes
+        # them; another's, or an overridden trace_backward, is called as is
+        own = getattr(ctx.pipeline.trace_backward, "__func__", None) is Pipeline.trace_backward
+        if own:
+            results = ctx.pipeline._backward(*args, **options, autograd=True)
+        else:
+            results = ctx.pipeline.trace_backward(*args, **options, eps=ctx.eps)
         points_grad = results["points_grad"].contiguous()
         attr_grad = results["attr_grad"].contiguous()
         sharpness_grad = results["sharpness_grad"].contiguous()
         if sharpness_grad is not None and isinstance(ctx.inv_s, torch.Tensor):
             sharpness_grad = sharpness_grad.to(ctx.inv_s.dtype).view_as(ctx.inv_s)
         ctx.errbox.point_error = results.get("point_error", None)
-        points_grad[~points_grad.isfinite()] = 0
-        attr_grad[~attr_grad.isfinite()] = 0
-        if sharpness_grad is not None:
+        if not own:
+            points_grad[~points_grad.isfinite()] = 0
+            attr_grad[~attr_grad.isfinite()] = 0
+        if not own or sharpness_grad.dtype != torch.float32:
+            # (a narrower type may have overflowed)
             sharpness_grad[~sharpness_grad.isfinite()] = 0
         del (ctx.rays, ctx.start_point, ctx.pipeline, ctx.rgba, ctx.points, ctx.attributes,
              ctx.point_adjacency, ctx.point_adjacency_offsets, ctx.depth_quantiles)
