@@ -261,7 +261,9 @@ typedef struct sdf_trace_plan {
     uint32_t walk_budget;     /* trips recorded per wavefront at most */
     const uint32_t *ray_order; /* device memory [num_rays], or NULL */
     void *grad_accum;          /* device memory, 256-byte aligned, or NULL */
-    size_t grad_accum_bytes;   /* >= sdf_grad_accum_bytes(sh_degree, num_points) */
+    size_t grad_accum_bytes;   /* >= sdf_grad_accum_bytes(sh_degree, num_points); with
+                                  8 * num_points (rounded up to 16) more, point errors
+                                  are summed there in fp64 */
     uint32_t scratch_ready;    /* backward: nonzero if `scratch` already holds this
                                   scene's offset table (the forward over the same
                                   scene filled it); the backward then skips

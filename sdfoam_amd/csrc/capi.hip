@@ -274,6 +274,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     rc = check_plan(plan, num_rays, settings->ray_image_width, rec, order);
     if (rc != SDF_OK) return rc;
     float *accum = nullptr;
+    double *error_sums = nullptr;
     if (plan && plan->grad_accum) {
         const size_t need = sdf_grad_accum_bytes(sh_degree, num_points);
         if (plan->grad_accum_bytes < need)
@@ -282,6 +283,9 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
         if ((reinterpret_cast<uintptr_t>(plan->grad_accum) & 255u) != 0)
             return fail(SDF_E_INVALID, "gradient accumulator must be 256-byte aligned");
         accum = static_cast<float *>(plan->grad_accum);
+        if (ray_error && point_error &&
+            plan->grad_accum_bytes >= need + error_sums_bytes(num_points))
+            error_sums = reinterpret_cast<double *>(static_cast<char *>(plan->grad_accum) + need);
     }
     const uint32_t outputs = plan ? plan->outputs : 0u;
     if ((outputs & SDF_OUTPUTS_FRESH) != 0 && (!accum || num_rays == 0))
@@ -300,7 +304,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (num_rays == 0) return SDF_OK;
     if (accum) {
         tbegin(SDF_KERNEL_GRAD_CLEAR, s);
-        e = launch_grad_clear(sh_degree, accum, num_points,
+        e = launch_grad_clear(sh_degree, accum, num_points, error_sums != nullptr,
                               (outputs & SDF_OUTPUTS_FRESH) ? sharpness_grad : nullptr, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "gradient accumulator clear");
@@ -328,6 +332,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     a.point_error = ray_error ? point_error : nullptr;
     a.sharpness_grad = sharpness_grad;
     a.accum = accum;
+    a.error_sums = error_sums;
     tbegin(SDF_KERNEL_BACKWARD, s);
     e = launch_backward(sh_degree, a, neus, false, half, s);
     tend(s);
@@ -335,7 +340,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (accum) {
         tbegin(SDF_KERNEL_GRAD_FINALIZE, s);
         e = launch_grad_finalize(sh_degree, accum, num_points, attribute_grad, points_grad,
-                                 a.point_error, sharpness_grad, outputs, half, s);
+                                 a.point_error, sharpness_grad, error_sums, outputs, half, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "gradient accumulator finalize");
     }

@@ -183,6 +183,9 @@ struct BwdArgs {
     // position x/y/z, point error), added into the outputs by
     // launch_grad_finalize; nullptr: atomics go to the outputs directly
     float *accum;
+    // behind the rows: the point errors' fp64 sums [N] (error_sums_bytes), or
+    // nullptr (the rows hold them)
+    double *error_sums;
     // walk statistics (STATS instantiation only)
     uint64_t *visit_hash;
     uint32_t *steps;
@@ -241,18 +244,26 @@ constexpr uint32_t accum_stride(int L) {
     return L <= 0 ? 8u : L <= 2 ? 32u : 64u;
 }
 
-// Clears num_points rows of the accumulator, and sharpness_grad[0] if given.
-hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, float *sharpness_grad,
-                             hipStream_t stream);
+// Bytes of the point errors' sums behind the accumulator's rows.
+__host__ inline uint64_t error_sums_bytes(uint32_t num_points) {
+    return (8ull * num_points + 15) / 16 * 16;
+}
+
+// Clears num_points rows of the accumulator, the point errors' sums behind
+// them (error_sums), and sharpness_grad[0] if given.
+hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, bool error_sums,
+                             float *sharpness_grad, hipStream_t stream);
 
 // attribute_grad [N, D] += rows[:, :D]; points_grad [N, 3] += rows[:, D:D+3];
-// point_error [N] += rows[:, D+3] (point_error may be nullptr).  attr_grad and
+// point_error [N] += rows[:, D+3], or error_sums where given (point_error may
+// be nullptr).  attr_grad and
 // point_error are fp16 when `half` (the sum is rounded once), else fp32.
 // outputs: SDF_OUTPUTS_* bits; with SDF_OUTPUTS_FINITE sharpness_grad[0] too
 // becomes 0 where it is not finite.
 hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, void *attr_grad,
                                 float *points_grad, void *point_error, float *sharpness_grad,
-                                uint32_t outputs, bool half, hipStream_t stream);
+                                const double *error_sums, uint32_t outputs, bool half,
+                                hipStream_t stream);
 
 hipError_t launch_backward(int L, const BwdArgs &a, bool neus, bool stats, bool half,
                            hipStream_t stream);

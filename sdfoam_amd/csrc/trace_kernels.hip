@@ -117,11 +117,10 @@ struct ContribTable {
     float alpha[SLOTS];
 };
 
-template <uint32_t SLOTS>
-__device__ __forceinline__ void contrib_clear(ContribTable<SLOTS> &ct) {
+__device__ __forceinline__ void contrib_clear(ContribTable<kContribSlots> &ct) {
     const uint32_t lane = lane_id();
 #pragma unroll
-    for (uint32_t k = 0; k < SLOTS / 64; ++k) {
+    for (uint32_t k = 0; k < kContribSlots / 64; ++k) {
         ct.tag[lane + 64u * k] = kContribFree;
         ct.w[lane + 64u * k] = 0.0f;
     }
@@ -152,15 +151,15 @@ __device__ __forceinline__ void contrib_add(ContribTable<SLOTS> &ct, uint32_t ce
 // flushes its occupied ones one per round, so the wave issues as many
 // atomic and store instructions as its busiest lane has occupied slots
 // (a few at C3) rather than one per slot position.
-template <typename AT, uint32_t SLOTS>
-__device__ __forceinline__ void contrib_flush(ContribTable<SLOTS> &ct, void *contribution,
-                                              float *alpha_out) {
-    static_assert(SLOTS / 64 <= 32, "one bit per slot of a lane");
+template <typename AT>
+__device__ __forceinline__ void contrib_flush(ContribTable<kContribSlots> &ct,
+                                              void *contribution, float *alpha_out) {
+    static_assert(kContribSlots / 64 <= 32, "one bit per slot of a lane");
     __builtin_amdgcn_wave_barrier();
     const uint32_t lane = lane_id();
     uint32_t occ = 0u;
 #pragma unroll
-    for (uint32_t k = 0; k < SLOTS / 64; ++k)
+    for (uint32_t k = 0; k < kContribSlots / 64; ++k)
         occ |= (ct.tag[lane + 64u * k] != kContribFree ? 1u : 0u) << k;
     while (__ballot(occ != 0u)) {
         if (occ) {
@@ -186,11 +185,9 @@ __device__ __forceinline__ void contrib_flush(ContribTable<SLOTS> &ct, void *con
 constexpr int kForwardWaves = 6;
 
 // CT: walk over the cell table (a.scene.cells) and read attribute rows from it.
-// HALF: the face scan's half-batch loads (walk_advance), for rays in an
-// explicit launch order (incoherent batches such as random training pixels).
-template <int L, bool NEUS, bool STATS, typename AT, bool CT = false, bool HALF = false>
+template <int L, bool NEUS, bool STATS, typename AT, bool CT = false>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(CT && !HALF && !STATS ? kForwardWaves : 1))) void
+__attribute__((amdgpu_waves_per_eu(CT && !STATS ? kForwardWaves : 1))) void
 forward_kernel(FwdArgs a) {
     constexpr uint32_t RB = CT ? cell_record_bytes(L, sizeof(AT)) : 0u;
     constexpr int nsh = (L + 1) * (L + 1);
@@ -244,14 +241,14 @@ forward_kernel(FwdArgs a) {
         uint2 entry = make_uint2(kWalkUnrecorded, 0u);
         if (ws.alive) {
             if constexpr (NEUS || STATS) {
-                walk_advance<true, STATS, false, false, RB, HALF>(a.scene, ray, max_steps, ws, si, wc);
+                walk_advance<true, STATS, false, false, RB>(a.scene, ray, max_steps, ws, si, wc);
                 entry = make_uint2(si.found ? si.next : kNoIndex,
                                    __builtin_bit_cast(uint32_t, si.t1));
             } else {
                 // the density backward walks in the unsafe mode: a step is
                 // recorded while that walk takes the same exit; from the first
                 // step where it would not, the backward scans for itself
-                walk_advance<true, false, false, true, RB, HALF>(a.scene, ray, max_steps, ws, si, wc);
+                walk_advance<true, false, false, true, RB>(a.scene, ray, max_steps, ws, si, wc);
                 if (si.agrees)
                     entry = make_uint2(si.found ? si.next : kNoIndex,
                                        __builtin_bit_cast(uint32_t, si.t1));
@@ -372,6 +369,407 @@ forward_kernel(FwdArgs a) {
     }
     store_attr4<AT>(a.rgba, ray_idx, make_float4(C0, C1, C2, 1.0f - T));
     if (a.num_intersections) a.num_intersections[ray_idx] = ws.n;
+}
+
+// ---------------------------------------------------------------------------
+// forward, G lanes per ray
+
+// With few rays the chip is not full and a walk's time is its latency: one
+// lane per ray scans a cell's ~16 faces one after another, in batches that each
+// wait for their loads (216 us for 44 trips at 64x64 rays and 4,104 cells, 4.7 us
+// a trip; 85 us with 16 lanes per ray).  Here G neighbouring lanes share a ray: they scan the faces G at a time (consecutive lanes read
+// consecutive table entries), combine the exits by DPP, and carry the same
+// walk state; three of them form one colour channel each.  The exit face is
+// the first minimum in row order as in walk_advance, every product and sum of
+// a step is the same one, so all outputs keep their bits.
+//
+// The walk record keeps its rows of 64 rays: a block is the G wavefronts of
+// one such row, which walk a chunk's 16 trips on their own and meet at its
+// end to claim the next one.  There they also empty the contribution table,
+// which the block shares: its sums are over 64 rays and 16 trips (over 64 and 8
+// in forward_kernel), so no sum takes more atomics, nor more roundings, than
+// with one lane per ray.
+template <int G>
+__device__ __forceinline__ uint32_t split_xor(uint32_t v, int step) {
+    // partner of each doubling step: lane ^ 1, lane ^ 2, then the mirror of
+    // 8 and of 16 lanes (groups of 4 and 8 hold one value by then)
+    switch (step) {
+    case 0: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xb1, 0xf, 0xf, false);
+    case 1: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4e, 0xf, 0xf, false);
+    case 2: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x141, 0xf, 0xf, false);
+    default: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x140, 0xf, 0xf, false);
+    }
+}
+
+// Position of ray r of wavefront w (of G) in its row of 64: for image rays a
+// compact part of the 8x8 tile, else consecutive.
+template <int G>
+__device__ __forceinline__ uint32_t split_position(uint32_t w, uint32_t r, bool image) {
+    if (!image) return w * (64u / G) + r;
+    if constexpr (G == 2) {
+        return w * 32u + r; // 8x4
+    } else if constexpr (G == 4) {
+        return ((w >> 1) * 4u + (r >> 2)) * 8u + (w & 1u) * 4u + (r & 3u); // 4x4
+    } else if constexpr (G == 8) {
+        return ((w >> 1) * 2u + (r >> 2)) * 8u + (w & 1u) * 4u + (r & 3u); // 4x2
+    } else {
+        return ((w >> 2) * 2u + (r >> 1)) * 8u + (w & 3u) * 2u + (r & 1u); // 2x2
+    }
+}
+
+// The row of 64 rays that block b of a split launch (of 4 * grid_blocks_for_
+// tiles blocks) takes: tiles go round robin over the XCDs, a tile's four rows
+// to the same one.
+__device__ __forceinline__ uint32_t split_row(uint32_t b) {
+    const uint32_t x = b % kXcds, k = b / kXcds;
+    return ((k / 4u) * kXcds + x) * 4u + k % 4u;
+}
+
+// ray at position l of row `row` (rows of ray_for_lane's wavefronts)
+__device__ __forceinline__ uint32_t ray_at(uint32_t row, uint32_t l, uint32_t num_rays,
+                                           uint32_t width, uint32_t num_tiles, bool &valid,
+                                           const uint32_t *__restrict__ order) {
+    const uint32_t t = row / 4u, w = row % 4u;
+    valid = false;
+    if (t >= num_tiles) return 0u;
+    if (width == 0 || order) {
+        const uint32_t i = row * 64u + l;
+        const uint32_t r = i < num_rays ? (order ? order[i] : i) : num_rays;
+        valid = r < num_rays;
+        return valid ? r : 0u;
+    }
+    const uint32_t height = num_rays / width;
+    const uint32_t tiles_x = (width + kTile - 1) / kTile;
+    const uint32_t x = (t % tiles_x) * kTile + (w & 1u) * 8u + (l & 7u);
+    const uint32_t y = (t / tiles_x) * kTile + (w >> 1) * 8u + (l >> 3);
+    valid = x < width && y < height;
+    return valid ? y * width + x : 0u;
+}
+
+// walk_advance<true, ...> over the cell table by the G lanes of a ray (all of
+// them active; the results are the same in each).  h: the lane's entries of
+// the first batch, loaded by the caller.
+template <int G, int U, bool DUAL, uint32_t RB>
+__device__ __forceinline__ void walk_advance_split(const SceneView &sc, const RayF &ray,
+                                                   uint32_t max_steps, uint32_t sub, uint2 *h,
+                                                   WalkState &ws, StepInfo &si) {
+    static_assert(G * U <= (int)kDiffPad, "a batch may over-read the table by its padding");
+    si.found = false;
+    si.agrees = true;
+    si.stepped = false;
+    si.t1 = ws.t0; // (no exit: what the walk record keeps beside its end mark)
+    ++ws.n;
+    if (ws.n > max_steps || ws.beg > ws.end || ws.end > sc.num_adj) {
+        ws.alive = false;
+        return;
+    }
+    const uint32_t nf = ws.end - ws.beg;
+    const float t0 = ws.t0;
+    float t1 = __builtin_bit_cast(float, 0x7f800000u);
+    float tmin_u = t1;
+    bool below = false;
+    uint32_t best = kNoIndex, bw = kDeltaNone;
+    float t1m = t1;
+    const float t0m = t0 * (1.0f - 0x1p-21f);
+    const float t0p = t0 * (1.0f + 0x1p-21f);
+    const uint2 *__restrict__ row = sc.diff + ws.beg;
+    for (uint32_t k0 = 0; k0 < nf; k0 += G * U) {
+        if (k0 != 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) h[u] = row[k0 + u * G + sub];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t k = k0 + u * G + sub;
+            const float dx = f16_to_f32(h[u].x);
+            const float dy = f16_to_f32(h[u].x >> 16);
+            const float dz = f16_to_f32(h[u].y);
+            const float fx = fmaf(dx, 0.5f, ws.xc[0]);
+            const float fy = fmaf(dy, 0.5f, ws.xc[1]);
+            const float fz = fmaf(dz, 0.5f, ws.xc[2]);
+            const float dp = sdf_dot3(dx, dy, dz, ray.dx, ray.dy, ray.dz);
+            const float num = sdf_dot3(fx - ray.ox, fy - ray.oy, fz - ray.oz, dx, dy, dz);
+            const bool pos = dp > 0.0f && k < nf;
+            // the division filter of walk_advance
+            const float lo = fmaf(t0m, dp, -0x1p-126f);
+            bool maybe = pos && num < fmaf(t1m, dp, 0x1p-126f) && num > lo;
+            if constexpr (DUAL) {
+                below = below || (pos && num < lo);
+                maybe = maybe || (pos && num >= lo && num <= fmaf(t0p, dp, 0x1p-126f));
+            }
+            if (maybe) {
+                const float t = num / dp;
+                if (t > t0 && t < t1) {
+                    t1 = t;
+                    t1m = fmaf(fabsf(t), 0x1p-21f, t);
+                    best = k;
+                    bw = h[u].y >> 16;
+                }
+                if constexpr (DUAL) tmin_u = fminf(tmin_u, t);
+            }
+        }
+    }
+    // the first minimum in row order: the smallest t, then the smallest k
+    uint32_t bl = below ? 1u : 0u;
+#pragma unroll
+    for (int s = 0; (1 << s) < G; ++s) {
+        const float ot = __builtin_bit_cast(float, split_xor<G>(__builtin_bit_cast(uint32_t, t1), s));
+        const uint32_t ob = split_xor<G>(best, s), ow = split_xor<G>(bw, s);
+        const bool take = ot < t1 || (ot == t1 && ob < best);
+        t1 = take ? ot : t1;
+        best = take ? ob : best;
+        bw = take ? ow : bw;
+        if constexpr (DUAL) {
+            bl |= split_xor<G>(bl, s);
+            tmin_u = fminf(tmin_u, __builtin_bit_cast(float, split_xor<G>(
+                                       __builtin_bit_cast(uint32_t, tmin_u), s)));
+        }
+    }
+    if constexpr (DUAL) si.agrees = !(bl != 0u || tmin_u <= t0);
+    if (best == kNoIndex) {
+        ws.alive = false;
+        return;
+    }
+    const uint32_t next = bw != kDeltaNone
+                              ? (uint32_t)((int32_t)ws.cell + (int32_t)(int16_t)(uint16_t)bw)
+                              : sc.adj[ws.beg + best];
+    if (next >= sc.num_points) {
+        ws.alive = false;
+        return;
+    }
+    si.found = true;
+    si.next = next;
+    si.t1 = t1;
+    load_cell<RB>(sc, next, si.xn, si.beg, si.end);
+    si.stepped = t1 > t0;
+}
+
+// slots of the block's contribution table: one per step between flushes
+constexpr uint32_t kSplitSlots = 64u * kChunkTrips;
+
+// The block's pending sums (all its threads, between two barriers).
+template <typename AT, int G>
+__device__ __forceinline__ void contrib_flush_block(ContribTable<kSplitSlots> &ct,
+                                                    void *contribution, float *alpha_out) {
+#pragma unroll
+    for (uint32_t k = 0; k < kSplitSlots / (64u * G); ++k) {
+        const uint32_t s = threadIdx.x + 64u * G * k;
+        const uint32_t c = ct.tag[s];
+        if (c == kContribFree) continue;
+        if (contribution) atomic_add_elem<AT>(contribution, c, ct.w[s]);
+        if (alpha_out) alpha_out[c] = ct.alpha[s];
+        ct.tag[s] = kContribFree;
+        ct.w[s] = 0.0f;
+    }
+}
+
+template <int L, bool NEUS, typename AT, int G>
+__global__ __launch_bounds__(64 * G) void forward_split_kernel(FwdArgs a) {
+    constexpr uint32_t RB = cell_record_bytes(L, sizeof(AT));
+    constexpr int nsh = (L + 1) * (L + 1);
+    constexpr int D = 1 + 3 * nsh;
+    constexpr int U = G >= 8 ? 32 / G : 4;
+    __shared__ ContribTable<kSplitSlots> ct;
+    // the block's chunk, its last trip and whether a ray walks on, for three
+    // chunks in turn (a slot is reset two chunks after its last reader)
+    __shared__ uint32_t blk_chunk[3], blk_end[3], blk_alive[3];
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+    const uint32_t sub = lane % G;
+    for (uint32_t k = threadIdx.x; k < kSplitSlots; k += 64u * G) {
+        ct.tag[k] = kContribFree;
+        ct.w[k] = 0.0f;
+    }
+    const uint32_t row_id = split_row(blockIdx.x);
+    const uint32_t pos = split_position<G>(wave, lane / G,
+                                           a.settings.ray_image_width != 0 && !a.order);
+    bool valid;
+    const uint32_t ray_idx = ray_at(row_id, pos, a.num_rays, a.settings.ray_image_width,
+                                    a.num_tiles, valid, a.order);
+    RayF ray = {};
+    if (valid) ray = load_ray(a.rays, ray_idx);
+    float sh[nsh];
+    sh_basis<L>(ray.dx, ray.dy, ray.dz, sh);
+    // with four lanes or more, three of them form one colour channel each
+    constexpr bool kByChannel = G >= 4;
+    const uint32_t ch = sub % 4u < 2u ? sub % 4u : 2u;
+    const float sha = a.sharpness[0];
+    const int32_t sdf_ch = a.settings.sdf_channel;
+    const bool neus_alpha = NEUS && sdf_ch >= 0;
+    const float thr = a.settings.weight_threshold;
+    const uint32_t Q = a.num_quantiles;
+    const float *rq = (valid && a.quantiles) ? a.quantiles + (uint64_t)ray_idx * Q : nullptr;
+    const uint64_t qbase = (uint64_t)ray_idx * Q;
+    const uint32_t max_steps = a.settings.max_intersections;
+    const bool sums = a.contribution || a.alpha_out;
+
+    float T = 1.0f, C = 0.0f, C1 = 0.0f, C2 = 0.0f; // by channel: C alone
+    uint32_t qi = 0;
+    float q = (rq && Q > 0) ? rq[0] : 0.0f;
+    WalkState ws;
+    walk_init<RB>(a.scene, valid ? a.start[ray_idx] : kNoIndex, ws);
+
+    uint64_t wslot = ~0ull; // this ray's entry in the first row of the chunk (~0: no chunk)
+
+    // one trip of the wavefront
+    auto advance = [&](uint32_t trip) {
+        StepInfo si;
+        si.stepped = false;
+        si.found = false;
+        uint2 entry = make_uint2(kWalkUnrecorded, 0u);
+        float rowv[kByChannel ? nsh : 1];
+        const AT *__restrict__ row = nullptr;
+        float s = 0.0f, chan = 0.0f;
+        if (ws.alive) {
+            // the faces' first batch, then the cell's row, all in flight at once
+            uint2 h[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) h[u] = make_uint2(0u, 0u);
+            if (ws.beg < ws.end && ws.end <= a.scene.num_adj) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) h[u] = a.scene.diff[ws.beg + u * G + sub];
+            }
+            row = reinterpret_cast<const AT *>(
+                reinterpret_cast<const char *>(a.scene.cells) + (uint64_t)ws.cell * RB +
+                kCellAttrByte);
+            s = (float)row[D - 1];
+            chan = neus_alpha ? (float)row[sdf_ch] : s;
+            if constexpr (kByChannel) {
+#pragma unroll
+                for (int j = 0; j < nsh; ++j) rowv[j] = (float)row[3 * j + ch];
+            }
+            walk_advance_split<G, U, !NEUS, RB>(a.scene, ray, max_steps, sub, h, ws, si);
+            if (NEUS || si.agrees)
+                entry = make_uint2(si.found ? si.next : kNoIndex,
+                                   __builtin_bit_cast(uint32_t, si.t1));
+            else if (si.found && a.scene.num_points < kWalkDiffers - 1u)
+                entry = make_uint2(si.next | kWalkDiffers, __builtin_bit_cast(uint32_t, si.t1));
+        }
+        float *col = nullptr;
+        if (wslot != ~0ull && trip < a.record.budget) {
+            const uint64_t i = wslot + (trip % kChunkTrips) * 64u;
+            if (sub == 0) record_store(a.record.entries + i, entry);
+            if (sub < 4u && (kByChannel || sub == 0))
+                col = reinterpret_cast<float *>(a.record.colors + i) + sub;
+        }
+        bool keep = true;
+        if (si.stepped) {
+            const uint32_t cell = ws.cell;
+            const float t0 = ws.t0, t1 = si.t1;
+            const float density = s;
+            const float dt = fmaxf(t1 - t0, 0.0f);
+            if (neus_alpha) {
+                const float phi = sdf_sigmoidf(-sha * chan);
+                s = sha * phi * (1.0f - phi);
+            }
+            const float alpha = 1.0f - sdf_expf(-s * dt);
+            const float w = T * alpha;
+            const float Tn = T * (1.0f - alpha);
+            const bool dense = NEUS || density > 1e-6f;
+            if constexpr (kByChannel) {
+                // sh_rgb_regs' sum for one channel
+                float v = 0.5f;
+#pragma unroll
+                for (int j = 0; j < nsh; ++j) v = fmaf(sh[j], rowv[j], v);
+                v = dense ? fmaxf(v, 0.0f) : 0.0f;
+                C = fmaf(w, v, C);
+                if (col) __builtin_nontemporal_store(sub == 3u ? chan : v, col);
+            } else {
+                float r, g, b;
+                if (dense) {
+                    sh_rgb_regs<L>(sh, row, r, g, b);
+                } else {
+                    r = g = b = 0.0f;
+                }
+                C = fmaf(w, r, C);
+                C1 = fmaf(w, g, C1);
+                C2 = fmaf(w, b, C2);
+                if (col) record_store(reinterpret_cast<float4 *>(col), make_float4(r, g, b, chan));
+            }
+            if (NEUS) {
+                const float drop = T - Tn;
+                if (drop > 1e-12f) {
+                    while (qi < Q && Tn < q) {
+                        float frac = (T - q) / drop;
+                        frac = fminf(1.0f, fmaxf(0.0f, frac));
+                        if (sub == 0) {
+                            a.depth[qbase + qi] = fmaf(frac, t1 - t0, t0);
+                            a.depth_indices[qbase + qi] = cell;
+                        }
+                        ++qi;
+                        if (qi < Q) q = rq[qi];
+                    }
+                }
+            } else {
+                while (qi < Q && Tn < q) {
+                    if (sub == 0) {
+                        a.depth[qbase + qi] = t0 + logf(T / q) / s;
+                        a.depth_indices[qbase + qi] = cell;
+                    }
+                    ++qi;
+                    if (qi < Q) q = rq[qi];
+                }
+            }
+            T = Tn;
+            keep = T > thr;
+            if (sums && sub == 0) contrib_add<AT>(ct, cell, w, alpha, a.contribution);
+        }
+        if (si.stepped && !keep) ws.alive = false;
+        if (ws.alive && si.found) walk_move(ws, si);
+    };
+
+    uint32_t *wtab = a.record.entries
+                         ? a.record.chunks + (uint64_t)row_id * chunk_slots(a.record.budget)
+                         : nullptr;
+    if (threadIdx.x < 3) blk_end[threadIdx.x] = blk_alive[threadIdx.x] = 0u;
+    __syncthreads(); // the table too is clear
+    if (__ballot(ws.alive) != 0ull && lane == 0) blk_alive[2] = 1u;
+    __syncthreads();
+    bool any = blk_alive[2] != 0u; // uniform over the block
+    for (uint32_t c = 0; any; ++c) {
+        const uint32_t first = c * kChunkTrips, now = c % 3u, reset = (c + 1u) % 3u;
+        if (threadIdx.x == 0) {
+            blk_chunk[now] = wtab && first < a.record.budget ? record_claim(a.record, wtab, c)
+                                                             : kNoIndex;
+            blk_end[reset] = 0u;
+            blk_alive[reset] = 0u;
+        }
+        __syncthreads(); // the last flush is done, the chunk is known
+        wslot = blk_chunk[now] == kNoIndex ? ~0ull
+                                           : (uint64_t)blk_chunk[now] * kChunkEntries + pos;
+        uint32_t trip = first;
+        while (trip < first + kChunkTrips && __ballot(ws.alive) != 0ull) advance(trip++);
+        const bool alive = __ballot(ws.alive) != 0ull;
+        if (lane == 0) {
+            atomicMax(&blk_end[now], trip);
+            if (alive) blk_alive[now] = 1u;
+        }
+        __syncthreads();
+        any = blk_alive[now] != 0u;
+        if (sums) contrib_flush_block<AT, G>(ct, a.contribution, a.alpha_out);
+        // the rows in which the block's other wavefronts still walked, and the
+        // one after the last
+        const uint32_t end = blk_end[now] + (blk_end[now] < first + kChunkTrips ? 1u : 0u);
+        for (; trip < end && trip < a.record.budget; ++trip) {
+            if (wslot != ~0ull && sub == 0)
+                record_store(a.record.entries + wslot + (trip % kChunkTrips) * 64u,
+                             make_uint2(kWalkUnrecorded, 0u));
+        }
+    }
+
+    if (!valid) return;
+    if (sub == 0) {
+        for (uint32_t k = qi; k < Q; ++k) {
+            a.depth[qbase + k] = -1.0f;
+            a.depth_indices[qbase + k] = kNoIndex;
+        }
+        if (a.num_intersections) a.num_intersections[ray_idx] = ws.n;
+    }
+    if constexpr (kByChannel) {
+        const float out = sub == 3u ? 1.0f - T : C;
+        if (sub < 4u) static_cast<AT *>(a.rgba)[4ull * ray_idx + sub] = (AT)out;
+    } else if (sub == 0) {
+        store_attr4<AT>(a.rgba, ray_idx, make_float4(C, C1, C2, 1.0f - T));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -514,7 +912,7 @@ struct OwnerLane {
 };
 
 template <int L, bool PE>
-__device__ __forceinline__ OwnerLane owner_lane(int last_ch) {
+__device__ __forceinline__ OwnerLane owner_lane(int last_ch, bool pe_sums) {
     using T = WaveTables<L, PE>;
     constexpr int nsh = (L + 1) * (L + 1);
     const int lane = (int)lane_id();
@@ -522,7 +920,7 @@ __device__ __forceinline__ OwnerLane owner_lane(int last_ch) {
     OwnerLane o;
     o.also_last = false;
     o.row_off = lane < D ? (uint32_t)lane : lane >= 60 ? (uint32_t)(D + lane - 60) : 0u;
-    o.row_active = lane < D || (lane >= 60 && lane < 63) || (lane == 63 && PE);
+    o.row_active = lane < D || (lane >= 60 && lane < 63) || (lane == 63 && PE && !pe_sums);
     if (lane < 3 * nsh) {
         o.y_base = (lane / 3) * kPitch;
         o.g_base = T::kRec + (lane % 3) * kPitch;
@@ -655,13 +1053,18 @@ __device__ __forceinline__ void publish_step(WaveTables<L, PE> &tb, StepEntries 
 // element of cell 0's row, so a group costs one address add.
 // !ACC: straight into attr_grad, points_grad (only when an entry of the
 // group flushed a position) and point_error.
+// error_sums (ACC, PE): the point errors' fp64 sums, [N], or NULL (they go to
+// the rows).  They are sums of one sign, and a cell that all rays cross gets one
+// term per wavefront: with fewer rays per wavefront there are more of them to
+// round, 1.2e-6 against 0.7e-6 of the sums at 400x400 rays in fp32.
 // ALSO_LAST: the last channel is an SH component too (sdf_channel < 3 nsh).
 template <int L, bool PE, typename AT, bool ACC, bool ALSO_LAST>
 __device__ __forceinline__ void grouped_pass_impl(StepEntries &e, const OwnerLane &ow,
                                                   WaveTables<L, PE> &tb, void *__restrict__ attr_grad,
                                                   void *__restrict__ point_error,
                                                   float *__restrict__ points_grad,
-                                                  float *__restrict__ row) {
+                                                  float *__restrict__ row,
+                                                  double *__restrict__ error_sums) {
     constexpr int D = 1 + 3 * (L + 1) * (L + 1);
     const uint32_t lane = lane_id();
     const float *last = tb.rec() + 3 * kPitch;
@@ -701,6 +1104,9 @@ __device__ __forceinline__ void grouped_pass_impl(StepEntries &e, const OwnerLan
         }
         if constexpr (ACC) {
             if (ow.row_active) atomicAdd(row + (uint64_t)c * accum_stride(L), acc);
+            if constexpr (PE) {
+                if (error_sums && lane == 63u) atomicAdd(error_sums + c, (double)acc);
+            }
         } else {
             const bool pos = flush_any != 0ull;
             if constexpr (sizeof(AT) == 4) {
@@ -732,6 +1138,7 @@ struct PassTarget {
     void *point_error;
     float *points_grad;
     float *row;         // accumulator: this lane's element of cell 0's row, or nullptr
+    double *error_sums; // beside the rows: the point errors' sums, or nullptr
     bool also_last;     // some owner lane adds the last channel to an SH component
 };
 
@@ -742,17 +1149,17 @@ __device__ __forceinline__ void grouped_pass(StepEntries &e, const OwnerLane &ow
     if (t.row) {
         if (t.also_last)
             grouped_pass_impl<L, PE, AT, true, true>(e, ow, tb, t.attr_grad, t.point_error,
-                                                     t.points_grad, t.row);
+                                                     t.points_grad, t.row, t.error_sums);
         else
             grouped_pass_impl<L, PE, AT, true, false>(e, ow, tb, t.attr_grad, t.point_error,
-                                                      t.points_grad, t.row);
+                                                      t.points_grad, t.row, t.error_sums);
     } else {
         if (t.also_last)
             grouped_pass_impl<L, PE, AT, false, true>(e, ow, tb, t.attr_grad, t.point_error,
-                                                      t.points_grad, t.row);
+                                                      t.points_grad, t.row, t.error_sums);
         else
             grouped_pass_impl<L, PE, AT, false, false>(e, ow, tb, t.attr_grad, t.point_error,
-                                                       t.points_grad, t.row);
+                                                       t.points_grad, t.row, t.error_sums);
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -764,6 +1171,7 @@ __device__ __forceinline__ PassTarget pass_target(const BwdArgs &a, const OwnerL
     t.point_error = a.point_error;
     t.points_grad = a.points_grad;
     t.row = a.accum ? a.accum + ow.row_off : nullptr;
+    t.error_sums = a.error_sums;
     t.also_last = __ballot(ow.also_last) != 0ull;
     return t;
 }
@@ -784,19 +1192,56 @@ __device__ __forceinline__ void tables_init(WaveTables<L, PE> &tb, const float *
     __builtin_amdgcn_wave_barrier();
 }
 
+// The ray of a backward's lane, its place in the walk record (row of 64 rays
+// and position in it) and its part of the ray (sub of G lanes).
+struct BackwardLane {
+    uint32_t ray, row, pos, sub;
+    bool valid;
+};
+
+// First wavefront of block b: tiles (4 G wavefronts, G blocks) go round robin
+// over the XCDs.
+template <int G>
+__device__ __forceinline__ uint32_t split_wave(uint32_t b) {
+    const uint32_t x = b % kXcds, k = b / kXcds;
+    return (((k / G) * kXcds + x) * G + k % G) * 4u;
+}
+
+template <int G>
+__device__ __forceinline__ BackwardLane backward_lane(const BwdArgs &a) {
+    BackwardLane b;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if constexpr (G == 1) {
+        b.ray = ray_for_lane<kBackwardChunk>(a.num_rays, a.settings.ray_image_width, a.num_tiles,
+                                             b.valid, a.order);
+        b.row = block_tile<kBackwardChunk>() * (kBlock / 64) + wave;
+        b.pos = lane;
+        b.sub = 0;
+    } else {
+        // wavefront `part` of the G that share a row of 64 rays
+        const uint32_t wv = split_wave<G>(blockIdx.x) + wave;
+        b.row = wv / G;
+        b.pos = split_position<G>(wv % G, lane / G,
+                                  a.settings.ray_image_width != 0 && !a.order);
+        b.sub = lane % G;
+        b.ray = ray_at(b.row, b.pos, a.num_rays, a.settings.ray_image_width, a.num_tiles, b.valid,
+                       a.order);
+    }
+    return b;
+}
+
 // ---------------------------------------------------------------------------
 // backward_sdf (src/tracing/pipeline.cu:267-550)
 
-template <int L, bool STATS, typename AT, bool PE = false>
+template <int L, bool STATS, typename AT, bool PE = false, int G = 1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 backward_sdf_kernel(BwdArgs a) {
     constexpr int nsh = (L + 1) * (L + 1);
     constexpr int D = 1 + 3 * nsh;
     __shared__ WaveTables<L, PE> tables[kBlock / 64];
-    bool valid;
-    const uint32_t ray_idx =
-        ray_for_lane<kBackwardChunk>(a.num_rays, a.settings.ray_image_width, a.num_tiles, valid,
-                                     a.order);
+    const BackwardLane bl = backward_lane<G>(a);
+    const bool valid = bl.valid;
+    const uint32_t ray_idx = bl.ray;
     const uint32_t lane = lane_id();
     WaveTables<L, PE> &tb = tables[threadIdx.x >> 6];
 
@@ -812,7 +1257,7 @@ backward_sdf_kernel(BwdArgs a) {
     const float sha = a.sharpness[0];
     const int32_t sdf_ch = a.settings.sdf_channel >= 0 ? a.settings.sdf_channel : D - 1;
     const bool write_sdf = a.settings.sdf_channel >= 0;
-    const OwnerLane owner = owner_lane<L, PE>(write_sdf ? sdf_ch : -1);
+    const OwnerLane owner = owner_lane<L, PE>(write_sdf ? sdf_ch : -1, a.error_sums != nullptr);
     const PassTarget target = pass_target<L>(a, owner);
     const float thr = a.settings.weight_threshold;
     const uint32_t Q = a.num_quantiles;
@@ -844,16 +1289,16 @@ backward_sdf_kernel(BwdArgs a) {
     WalkCounters wc = {0u, 0u, 0ull, 0ull};
     // replay of the forward's walk record: while this lane's entries are
     // recorded, the step is read instead of scanned; from the first
-    // unrecorded (or out-of-range) entry on, the lane scans.  wslot: this
-    // lane's entry in the first row of the trip's chunk (~0: no chunk).
+    // unrecorded (or out-of-range) entry on, the lane scans
     const uint32_t *wtab = nullptr;
-    uint64_t wslot = ~0ull;
     bool replaying = false;
+    uint64_t wslot = ~0ull;
     if (!STATS && a.record.entries) {
-        wtab = walk_record_table<kBackwardChunk>(a.record);
+        wtab = a.record.chunks + (uint64_t)bl.row * chunk_slots(a.record.budget);
         replaying = true;
     }
     uint32_t trip = 0;
+    uint32_t turn = 0; // the ray's steps: the lane that publishes them in turn (G > 1)
     StepEntries ents; // steps whose updates are not applied yet
     entries_init(ents);
 
@@ -866,7 +1311,7 @@ backward_sdf_kernel(BwdArgs a) {
         bool replayed = false;
         if (wtab && trip < a.record.budget && trip % kChunkTrips == 0) {
             const uint32_t c = wtab[trip / kChunkTrips];
-            wslot = c == kNoIndex ? ~0ull : (uint64_t)c * kChunkEntries + lane;
+            wslot = c == kNoIndex ? ~0ull : (uint64_t)c * kChunkEntries + bl.pos;
         }
         if (ws.alive) {
             uint2 e = make_uint2(kWalkUnrecorded, 0u);
@@ -982,8 +1427,9 @@ backward_sdf_kernel(BwdArgs a) {
             // steps go out every kWindow trips
             if (ents.pend && (si.stepped || !ws.alive))
                 complete_entry<L, PE>(ents, si.stepped && flush, flush_g, tb);
-            if (trip % kWindow == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
-            if (si.stepped) publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dsdf, pe);
+            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
+            if (si.stepped && (G == 1 || turn++ % G == bl.sub))
+                publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dsdf, pe);
         }
         if (ws.alive && si.found) walk_move(ws, si);
     }
@@ -1003,7 +1449,7 @@ backward_sdf_kernel(BwdArgs a) {
         }
     } else {
         if (a.sharpness_grad) {
-            const float v = wave_sum(sharp_acc);
+            const float v = wave_sum(G == 1 || bl.sub == 0 ? sharp_acc : 0.0f);
             if (lane == 0 && v != 0.0f) atomicAdd(a.sharpness_grad, v);
         }
     }
@@ -1011,16 +1457,15 @@ backward_sdf_kernel(BwdArgs a) {
 
 // backward, density mode (src/tracing/pipeline.cu:553-791); the walk runs in
 // the reference's unsafe mode (no t > t0 test, :782-790).
-template <int L, bool STATS, typename AT, bool PE = false>
+template <int L, bool STATS, typename AT, bool PE = false, int G = 1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 backward_density_kernel(BwdArgs a) {
     constexpr int nsh = (L + 1) * (L + 1);
     constexpr int D = 1 + 3 * nsh;
     __shared__ WaveTables<L, PE> tables[kBlock / 64];
-    bool valid;
-    const uint32_t ray_idx =
-        ray_for_lane<kBackwardChunk>(a.num_rays, a.settings.ray_image_width, a.num_tiles, valid,
-                                     a.order);
+    const BackwardLane bl = backward_lane<G>(a);
+    const bool valid = bl.valid;
+    const uint32_t ray_idx = bl.ray;
     const uint32_t lane = lane_id();
     WaveTables<L, PE> &tb = tables[threadIdx.x >> 6];
 
@@ -1033,7 +1478,7 @@ backward_density_kernel(BwdArgs a) {
     }
     const float *sh = tb.y() + lane; // this ray's SH basis, in LDS (stride kPitch)
 
-    const OwnerLane owner = owner_lane<L, PE>(D - 1);
+    const OwnerLane owner = owner_lane<L, PE>(D - 1, a.error_sums != nullptr);
     const PassTarget target = pass_target<L>(a, owner);
     const float thr = a.settings.weight_threshold;
     const uint32_t Q = a.num_quantiles;
@@ -1075,10 +1520,11 @@ backward_density_kernel(BwdArgs a) {
     const uint32_t *wtab = nullptr;
     bool replaying = false;
     if (!STATS && a.record.entries) {
-        wtab = walk_record_table<kBackwardChunk>(a.record);
+        wtab = a.record.chunks + (uint64_t)bl.row * chunk_slots(a.record.budget);
         replaying = true;
     }
     uint32_t trip = 0;
+    uint32_t turn = 0; // the ray's steps: the lane that publishes them in turn (G > 1)
     // ridx: the forward trip whose entry the lane reads next.  After an entry
     // marked kWalkDiffers the lane scans (`seeking`) until its walk stands
     // where the forward stood after one of that entry's first kSeekWindow
@@ -1099,7 +1545,7 @@ backward_density_kernel(BwdArgs a) {
         if (ws.alive) {
             uint2 e = make_uint2(kWalkUnrecorded, 0u);
             if (replaying && !seeking && ridx < a.record.budget) {
-                const uint64_t i = record_slot(a.record, wtab, ridx, lane);
+                const uint64_t i = record_slot(a.record, wtab, ridx, bl.pos);
                 if (i != ~0ull) {
                     e = record_load(a.record.entries + i);
                     rc4 = record_load(a.record.colors + i);
@@ -1212,8 +1658,9 @@ backward_density_kernel(BwdArgs a) {
         if constexpr (!STATS) {
             if (ents.pend && (si.stepped || !ws.alive))
                 complete_entry<L, PE>(ents, si.stepped && flush, flush_g, tb);
-            if (trip % kWindow == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
-            if (si.stepped) publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dds, pe);
+            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
+            if (si.stepped && (G == 1 || turn++ % G == bl.sub))
+                publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dds, pe);
         }
         if (ws.alive && si.found) walk_move(ws, si);
         if (seeking && ws.alive) {
@@ -1223,7 +1670,7 @@ backward_density_kernel(BwdArgs a) {
             for (uint32_t k = 0; k < kSeekWindow; ++k) {
                 const uint32_t f = ridx - 1u + k;
                 if (f >= a.record.budget) break;
-                const uint64_t i = record_slot(a.record, wtab, f, lane);
+                const uint64_t i = record_slot(a.record, wtab, f, bl.pos);
                 if (i == ~0ull) break;
                 const uint2 fe = record_load(a.record.entries + i);
                 if (fe.x == kNoIndex || fe.x == kWalkUnrecorded) break;
@@ -1258,18 +1705,78 @@ backward_density_kernel(BwdArgs a) {
 static inline dim3 grid_for(uint64_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
 
 
+// Lanes per ray of the forward and the backward.  Few rays leave the chip idle
+// and a walk's time is its latency: more lanes shorten it.  More rays fill it,
+// and the work that the lanes of a ray repeat costs more than it gives; the
+// sooner, the more rays there are per cell (their wavefronts then share cells,
+// and end together).  The lines are where the two sides met over six scenes of
+// 4k to 3M points (ms, forward / backward):
+//   rays / points      1 lane       2            4            8            16
+//   6.7k / 300k      2.08/2.30     -/1.38     1.04/0.91    0.84/0.69    0.82/0.58
+//   20k batch / 300k 1.63/1.30     -/0.87     0.85/0.73    0.76/0.68    1.00/0.79
+//   65k batch / 200k 1.89/2.27  1.36/1.96     1.08/1.72    1.39/1.91    2.04/2.28
+//   307k / 1M        4.26/4.07  2.89/2.67     2.79/2.63    3.36/3.52    5.53/5.86
+//   750k / 1M        4.76/4.74  4.47/4.02     4.75/4.80
+//   1M batch / 2M    18.4/22.2  17.5/19.2     17.1/20.3
+//   1.9M / 1M        7.18/7.50  9.15/7.09     10.6/10.6
+//   32k / 4k         0.34/0.21  0.26/0.15     0.24/0.14    0.28/0.16    0.34/0.22
+//   90k / 10k        0.45/0.31  0.39/0.28     0.41/0.33    0.50/0.49    0.74/0.79
+//   202k / 30k       0.66/0.58  0.75/0.59     0.77/0.75    1.07/1.23    1.84/2.13
+//   900k / 30k       1.14/1.40  1.44/1.54     1.84/2.41
+// (two lanes shorten the backward even where the chip is full: 32 rays over six
+// trips meet fewer distinct cells than 64 rays over three).
+static int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered) {
+    if (num_rays < 2ull * num_points) {
+        if (num_rays <= 16384u) return 16;
+        if (num_rays <= 49152u) return 8;
+        if (ordered || num_rays <= 400000u) return 4;
+        return num_rays <= 800000u ? 2 : 1;
+    }
+    if (num_rays <= 8192u) return 8;
+    if (num_rays <= 65536u) return 4;
+    if (ordered) return num_rays < 16ull * num_points ? 2 : 1;
+    return num_rays <= 163840u ? 2 : 1;
+}
+
+static int backward_lanes(uint32_t num_rays, uint32_t num_points) {
+    if (num_rays < 2ull * num_points) {
+        if (num_rays <= 16384u) return 16;
+        if (num_rays <= 49152u) return 8;
+        return num_rays <= 330000u ? 4 : 2;
+    }
+    if (num_rays <= 8192u) return 8;
+    if (num_rays <= 40960u) return 4;
+    return num_rays < 16ull * num_points ? 2 : 1;
+}
+
+template <int L, typename AT, int G>
+static hipError_t launch_forward_split(const FwdArgs &a, bool neus, hipStream_t stream) {
+    const dim3 grid(4 * grid_blocks_for_tiles(a.num_tiles)); // one block per 64 rays
+    if (neus) {
+        hipLaunchKernelGGL((forward_split_kernel<L, true, AT, G>), grid, dim3(64 * G), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((forward_split_kernel<L, false, AT, G>), grid, dim3(64 * G), 0, stream, a);
+    }
+    return hipGetLastError();
+}
+
 template <int L, typename AT>
 static hipError_t launch_forward_L(const FwdArgs &a, bool neus, bool stats, hipStream_t stream) {
     const dim3 grid(grid_blocks_for_tiles(a.num_tiles));
     const bool ct = a.scene.cells != nullptr;
-    // rays in an explicit order are an incoherent batch: half-batch face loads
-    const bool half = a.order != nullptr;
+    // (fp16 sums keep their roundings: each atomic of theirs rounds to 11 bits)
+    if (ct && !stats && !(sizeof(AT) == 2 && a.contribution)) {
+        switch (forward_lanes(a.num_rays, a.scene.num_points, a.order != nullptr)) {
+        case 16: return launch_forward_split<L, AT, 16>(a, neus, stream);
+        case 8: return launch_forward_split<L, AT, 8>(a, neus, stream);
+        case 4: return launch_forward_split<L, AT, 4>(a, neus, stream);
+        case 2: return launch_forward_split<L, AT, 2>(a, neus, stream);
+        default: break;
+        }
+    }
     if (neus) {
         if (stats) {
             hipLaunchKernelGGL((forward_kernel<L, true, true, AT>), grid, dim3(kBlock), 0, stream, a);
-        } else if (ct && half) {
-            hipLaunchKernelGGL((forward_kernel<L, true, false, AT, true, true>), grid, dim3(kBlock),
-                               0, stream, a);
         } else if (ct) {
             hipLaunchKernelGGL((forward_kernel<L, true, false, AT, true>), grid, dim3(kBlock), 0,
                                stream, a);
@@ -1279,9 +1786,6 @@ static hipError_t launch_forward_L(const FwdArgs &a, bool neus, bool stats, hipS
     } else {
         if (stats) {
             hipLaunchKernelGGL((forward_kernel<L, false, true, AT>), grid, dim3(kBlock), 0, stream, a);
-        } else if (ct && half) {
-            hipLaunchKernelGGL((forward_kernel<L, false, false, AT, true, true>), grid,
-                               dim3(kBlock), 0, stream, a);
         } else if (ct) {
             hipLaunchKernelGGL((forward_kernel<L, false, false, AT, true>), grid, dim3(kBlock), 0,
                                stream, a);
@@ -1463,31 +1967,47 @@ hipError_t launch_forward(int L, const FwdArgs &a, bool neus, bool stats, bool h
                 : launch_forward_T<float>(L, a, neus, stats, stream);
 }
 
+template <int L, typename AT, int G>
+static hipError_t launch_backward_G(const BwdArgs &a, bool neus, hipStream_t stream) {
+    // one block per tile, or 4 wavefronts of the G that share a row of 64 rays
+    const uint32_t tiles = grid_blocks_for_tiles(a.num_tiles);
+    const dim3 grid(tiles * G);
+    // PE: entries carry the point error (a larger LDS table per wave)
+    const bool pe = a.point_error != nullptr;
+    if (neus && pe) {
+        hipLaunchKernelGGL((backward_sdf_kernel<L, false, AT, true, G>), grid, dim3(kBlock), 0,
+                           stream, a);
+    } else if (neus) {
+        hipLaunchKernelGGL((backward_sdf_kernel<L, false, AT, false, G>), grid, dim3(kBlock), 0,
+                           stream, a);
+    } else if (pe) {
+        hipLaunchKernelGGL((backward_density_kernel<L, false, AT, true, G>), grid, dim3(kBlock), 0,
+                           stream, a);
+    } else {
+        hipLaunchKernelGGL((backward_density_kernel<L, false, AT, false, G>), grid, dim3(kBlock),
+                           0, stream, a);
+    }
+    return hipGetLastError();
+}
+
 template <int L, typename AT>
 static hipError_t launch_backward_L(const BwdArgs &a, bool neus, bool stats, hipStream_t stream) {
+    if (!stats) {
+        // (fp16 gradients without the accumulator keep their roundings)
+        const bool keep = sizeof(AT) == 2 && !a.accum;
+        switch (keep ? 1 : backward_lanes(a.num_rays, a.scene.num_points)) {
+        case 16: return launch_backward_G<L, AT, 16>(a, neus, stream);
+        case 8: return launch_backward_G<L, AT, 8>(a, neus, stream);
+        case 4: return launch_backward_G<L, AT, 4>(a, neus, stream);
+        case 2: return launch_backward_G<L, AT, 2>(a, neus, stream);
+        default: return launch_backward_G<L, AT, 1>(a, neus, stream);
+        }
+    }
     const dim3 grid(grid_blocks_for_tiles(a.num_tiles));
-    // PE: entries carry the point error (a larger LDS table per wave)
-    const bool pe = !stats && a.point_error != nullptr;
     if (neus) {
-        if (stats) {
-            hipLaunchKernelGGL((backward_sdf_kernel<L, true, AT>), grid, dim3(kBlock), 0, stream, a);
-        } else if (pe) {
-            hipLaunchKernelGGL((backward_sdf_kernel<L, false, AT, true>), grid, dim3(kBlock), 0,
-                               stream, a);
-        } else {
-            hipLaunchKernelGGL((backward_sdf_kernel<L, false, AT>), grid, dim3(kBlock), 0, stream, a);
-        }
+        hipLaunchKernelGGL((backward_sdf_kernel<L, true, AT>), grid, dim3(kBlock), 0, stream, a);
     } else {
-        if (stats) {
-            hipLaunchKernelGGL((backward_density_kernel<L, true, AT>), grid, dim3(kBlock), 0, stream,
-                               a);
-        } else if (pe) {
-            hipLaunchKernelGGL((backward_density_kernel<L, false, AT, true>), grid, dim3(kBlock), 0,
-                               stream, a);
-        } else {
-            hipLaunchKernelGGL((backward_density_kernel<L, false, AT>), grid, dim3(kBlock), 0,
-                               stream, a);
-        }
+        hipLaunchKernelGGL((backward_density_kernel<L, true, AT>), grid, dim3(kBlock), 0, stream, a);
     }
     return hipGetLastError();
 }
@@ -1538,7 +2058,7 @@ template <int L, typename AT, bool FRESH>
 __global__ __launch_bounds__(kBlock) void grad_finalize_kernel(
     const float4 *__restrict__ rows, uint32_t num_points, AT *__restrict__ attr_grad,
     float *__restrict__ points_grad, AT *__restrict__ point_error,
-    float *__restrict__ sharpness_grad, bool finite) {
+    float *__restrict__ sharpness_grad, const double *__restrict__ error_sums, bool finite) {
     constexpr uint32_t S4 = accum_stride(L) / 4;
     constexpr uint32_t D = 1 + 3 * (L + 1) * (L + 1);
     constexpr uint32_t Q = (D + 4 + 3) / 4; // quads of a row that hold data
@@ -1553,8 +2073,9 @@ __global__ __launch_bounds__(kBlock) void grad_finalize_kernel(
         const uint32_t q = (uint32_t)(t % S4);
         if (q >= Q) continue;
         const float4 v4 = rows[t];
-        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+        float v[4] = {v4.x, v4.y, v4.z, v4.w};
         const uint64_t c = t / S4;
+        if (error_sums && q == (D + 3) / 4) v[(D + 3) % 4] = (float)error_sums[c];
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
             const uint32_t j = 4u * q + k;
@@ -1588,10 +2109,11 @@ static inline dim3 accum_grid(uint64_t threads) {
     return dim3((unsigned)(b < kAccumBlocks ? (b ? b : 1) : kAccumBlocks));
 }
 
-hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, float *sharpness_grad,
-                             hipStream_t stream) {
+hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, bool error_sums,
+                             float *sharpness_grad, hipStream_t stream) {
     if (L < 0 || L > 3) return hipErrorInvalidValue;
-    const uint64_t n4 = (uint64_t)num_points * accum_stride(L) / 4;
+    const uint64_t n4 = (uint64_t)num_points * accum_stride(L) / 4 +
+                        (error_sums ? error_sums_bytes(num_points) / 16 : 0);
     hipLaunchKernelGGL(grad_clear_kernel, accum_grid(n4), dim3(kBlock), 0, stream,
                        reinterpret_cast<float4 *>(accum), n4, sharpness_grad);
     return hipGetLastError();
@@ -1600,8 +2122,8 @@ hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, float *sh
 template <int L, typename AT>
 static hipError_t launch_grad_finalize_L(const float *accum, uint32_t num_points, void *attr_grad,
                                          float *points_grad, void *point_error,
-                                         float *sharpness_grad, uint32_t outputs,
-                                         hipStream_t stream) {
+                                         float *sharpness_grad, const double *error_sums,
+                                         uint32_t outputs, hipStream_t stream) {
     const dim3 grid = accum_grid((uint64_t)num_points * accum_stride(L) / 4);
     const float4 *rows = reinterpret_cast<const float4 *>(accum);
     AT *ag = static_cast<AT *>(attr_grad);
@@ -1609,24 +2131,27 @@ static hipError_t launch_grad_finalize_L(const float *accum, uint32_t num_points
     const bool finite = (outputs & SDF_OUTPUTS_FINITE) != 0;
     if (outputs & SDF_OUTPUTS_FRESH) {
         hipLaunchKernelGGL((grad_finalize_kernel<L, AT, true>), grid, dim3(kBlock), 0, stream, rows,
-                           num_points, ag, points_grad, pe, sharpness_grad, finite);
+                           num_points, ag, points_grad, pe, sharpness_grad, error_sums, finite);
     } else {
         hipLaunchKernelGGL((grad_finalize_kernel<L, AT, false>), grid, dim3(kBlock), 0, stream, rows,
-                           num_points, ag, points_grad, pe, nullptr, false);
+                           num_points, ag, points_grad, pe, nullptr, error_sums, false);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, void *attr_grad,
                                 float *points_grad, void *point_error, float *sharpness_grad,
-                                uint32_t outputs, bool half, hipStream_t stream) {
-#define SDF_FINALIZE(N)                                                                          \
-    case N:                                                                                      \
-        return half ? launch_grad_finalize_L<N, _Float16>(accum, num_points, attr_grad,          \
-                                                          points_grad, point_error,              \
-                                                          sharpness_grad, outputs, stream)       \
-                    : launch_grad_finalize_L<N, float>(accum, num_points, attr_grad, points_grad, \
-                                                       point_error, sharpness_grad, outputs,     \
+                                const double *error_sums, uint32_t outputs, bool half,
+                                hipStream_t stream) {
+#define SDF_FINALIZE(N)                                                                        \
+    case N:                                                                                    \
+        return half ? launch_grad_finalize_L<N, _Float16>(accum, num_points, attr_grad,        \
+                                                          points_grad, point_error,            \
+                                                          sharpness_grad, error_sums, outputs, \
+                                                          stream)                              \
+                    : launch_grad_finalize_L<N, float>(accum, num_points, attr_grad,           \
+                                                       points_grad, point_error,               \
+                                                       sharpness_grad, error_sums, outputs,    \
                                                        stream)
     switch (L) {
         SDF_FINALIZE(0);

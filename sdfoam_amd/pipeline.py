@@ -699,6 +699,8 @@ class Pipeline:
         accum = None
         if grad_accum and num_rays > 0:
             accum_bytes = int(_lib.lib().sdf_grad_accum_bytes(self._sh_degree, num_points))
+            if return_error:
+                accum_bytes += -(-8 * num_points // 16) * 16  # its fp64 sums
             accum = torch.empty(accum_bytes + 256, dtype=torch.uint8, device=dev)
             desc.grad_accum = (accum.data_ptr() + 255) & ~255
             desc.grad_accum_bytes = accum_bytes
