@@ -211,6 +211,23 @@ int sdf_trace_benchmark(int sh_degree, const sdf_trace_settings *settings,
                         uint32_t *output_rgba, const float *sharpness,
                         void *stream);
 
+/* sdf_trace_benchmark with scratch for the frame's cell table and a padded
+ * copy of the offset table: the same image, sooner.  scratch: 256-byte
+ * aligned, or NULL (the caller's arrays are walked).  The size is 0 where the
+ * frame has too few pixels for the tables to pay. */
+size_t sdf_trace_benchmark_scratch_bytes(int sh_degree, int attr_type,
+                                         uint32_t num_points,
+                                         uint32_t adjacency_size,
+                                         uint32_t width, uint32_t height);
+int sdf_trace_benchmark_planned(
+    int sh_degree, const sdf_trace_settings *settings, uint32_t num_points,
+    const float *points, const float *attributes, uint32_t adjacency_size,
+    const uint32_t *point_adjacency, const uint32_t *point_adjacency_offsets,
+    const uint16_t *adjacent_diff, size_t adjacent_diff_entries,
+    const sdf_camera *camera, const sdf_visualization *vis,
+    const uint32_t *start_point_index, uint32_t *output_rgba,
+    const float *sharpness, void *scratch, size_t scratch_bytes, void *stream);
+
 /* ---- trace plan (no counterpart in the reference) ---------------------- *
  * Two optional aids for a forward and the backward over the same rays, start
  * points, scene and settings.  Results are identical with and without them.

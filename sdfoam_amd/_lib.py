@@ -30,6 +30,8 @@ EXPORTS = (
     "sdf_trace_forward_noalloc",
     "sdf_trace_backward",
     "sdf_trace_benchmark",
+    "sdf_trace_benchmark_scratch_bytes",
+    "sdf_trace_benchmark_planned",
     "sdf_walk_record_bytes",
     "sdf_walk_record_pool_bytes",
     "sdf_walk_record_full_chunks",
@@ -182,6 +184,12 @@ def lib() -> C.CDLL:
     L.sdf_trace_benchmark.argtypes = [
         C.c_int, C.POINTER(TraceSettings), U32, P, P, U32, P, P, P, SZ, C.POINTER(Camera),
         C.POINTER(Visualization), P, P, P, P]
+    L.sdf_trace_benchmark_scratch_bytes.restype = SZ
+    L.sdf_trace_benchmark_scratch_bytes.argtypes = [C.c_int, C.c_int, U32, U32, U32, U32]
+    L.sdf_trace_benchmark_planned.restype = C.c_int
+    L.sdf_trace_benchmark_planned.argtypes = [
+        C.c_int, C.POINTER(TraceSettings), U32, P, P, U32, P, P, P, SZ, C.POINTER(Camera),
+        C.POINTER(Visualization), P, P, P, P, SZ, P]
     L.sdf_walk_record_bytes.restype = SZ
     L.sdf_walk_record_bytes.argtypes = [U32, U32, U32]
     L.sdf_walk_record_pool_bytes.restype = SZ

@@ -197,7 +197,7 @@ struct BwdArgs {
 
 // Inference render (Pipeline::trace_benchmark): rays cast per pixel.
 struct RenderArgs {
-    SceneView scene; // diff: the caller's table, no padding
+    SceneView scene; // diff: the caller's table, no padding; or, with cells, its padded copy
     sdf_trace_settings settings;
     float position[3], forward[3], right[3], up[3];
     float fov, focal; // focal = 1 / tan(fov / 2)
@@ -234,9 +234,14 @@ hipError_t launch_forward(int L, const FwdArgs &a, bool neus, bool stats, bool h
 // Fills the fp16 offset table `diff` (as launch_prefetch_diff) and the cell
 // table (cell_record_bytes(L, attribute size) per cell) from sc's points,
 // adjacency, offsets and attributes, in one pass, and zeroes contribution
-// (attribute type) and alpha [N] where they are given.
+// (attribute type) and alpha [N] where they are given.  given: a caller's
+// offset table [num_adj] to take the offsets from, or nullptr.
 hipError_t launch_scene_prep(int L, bool half, const SceneView &sc, uint32_t *cells, uint2 *diff,
-                             void *contribution, float *alpha, hipStream_t stream);
+                             void *contribution, float *alpha, const uint2 *given,
+                             hipStream_t stream);
+// Lanes per ray (1 to 16) of a walk over the cell table; `ordered`: rays in an
+// explicit launch order.
+int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered);
 // Floats per cell row of the backward's gradient accumulator: the next
 // power of two >= D + 4 (attribute row, position, point error), at least 8,
 // so that a row spans the fewest 64-byte segments.

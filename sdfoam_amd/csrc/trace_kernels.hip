@@ -15,6 +15,7 @@
 // Each per-element contribution is the same fp32 product the reference
 // forms; only the order of the sums differs (fp32 atomics have no order).
 #include "trace_kernels.h"
+#include "trace_split.h"
 
 #include <algorithm>
 
@@ -389,161 +390,6 @@ forward_kernel(FwdArgs a) {
 // which the block shares: its sums are over 64 rays and 16 trips (over 64 and 8
 // in forward_kernel), so no sum takes more atomics, nor more roundings, than
 // with one lane per ray.
-template <int G>
-__device__ __forceinline__ uint32_t split_xor(uint32_t v, int step) {
-    // partner of each doubling step: lane ^ 1, lane ^ 2, then the mirror of
-    // 8 and of 16 lanes (groups of 4 and 8 hold one value by then)
-    switch (step) {
-    case 0: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xb1, 0xf, 0xf, false);
-    case 1: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4e, 0xf, 0xf, false);
-    case 2: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x141, 0xf, 0xf, false);
-    default: return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x140, 0xf, 0xf, false);
-    }
-}
-
-// Position of ray r of wavefront w (of G) in its row of 64: for image rays a
-// compact part of the 8x8 tile, else consecutive.
-template <int G>
-__device__ __forceinline__ uint32_t split_position(uint32_t w, uint32_t r, bool image) {
-    if (!image) return w * (64u / G) + r;
-    if constexpr (G == 2) {
-        return w * 32u + r; // 8x4
-    } else if constexpr (G == 4) {
-        return ((w >> 1) * 4u + (r >> 2)) * 8u + (w & 1u) * 4u + (r & 3u); // 4x4
-    } else if constexpr (G == 8) {
-        return ((w >> 1) * 2u + (r >> 2)) * 8u + (w & 1u) * 4u + (r & 3u); // 4x2
-    } else {
-        return ((w >> 2) * 2u + (r >> 1)) * 8u + (w & 3u) * 2u + (r & 1u); // 2x2
-    }
-}
-
-// The row of 64 rays that block b of a split launch (of 4 * grid_blocks_for_
-// tiles blocks) takes: tiles go round robin over the XCDs, a tile's four rows
-// to the same one.
-__device__ __forceinline__ uint32_t split_row(uint32_t b) {
-    const uint32_t x = b % kXcds, k = b / kXcds;
-    return ((k / 4u) * kXcds + x) * 4u + k % 4u;
-}
-
-// ray at position l of row `row` (rows of ray_for_lane's wavefronts)
-__device__ __forceinline__ uint32_t ray_at(uint32_t row, uint32_t l, uint32_t num_rays,
-                                           uint32_t width, uint32_t num_tiles, bool &valid,
-                                           const uint32_t *__restrict__ order) {
-    const uint32_t t = row / 4u, w = row % 4u;
-    valid = false;
-    if (t >= num_tiles) return 0u;
-    if (width == 0 || order) {
-        const uint32_t i = row * 64u + l;
-        const uint32_t r = i < num_rays ? (order ? order[i] : i) : num_rays;
-        valid = r < num_rays;
-        return valid ? r : 0u;
-    }
-    const uint32_t height = num_rays / width;
-    const uint32_t tiles_x = (width + kTile - 1) / kTile;
-    const uint32_t x = (t % tiles_x) * kTile + (w & 1u) * 8u + (l & 7u);
-    const uint32_t y = (t / tiles_x) * kTile + (w >> 1) * 8u + (l >> 3);
-    valid = x < width && y < height;
-    return valid ? y * width + x : 0u;
-}
-
-// walk_advance<true, ...> over the cell table by the G lanes of a ray (all of
-// them active; the results are the same in each).  h: the lane's entries of
-// the first batch, loaded by the caller.
-template <int G, int U, bool DUAL, uint32_t RB>
-__device__ __forceinline__ void walk_advance_split(const SceneView &sc, const RayF &ray,
-                                                   uint32_t max_steps, uint32_t sub, uint2 *h,
-                                                   WalkState &ws, StepInfo &si) {
-    static_assert(G * U <= (int)kDiffPad, "a batch may over-read the table by its padding");
-    si.found = false;
-    si.agrees = true;
-    si.stepped = false;
-    si.t1 = ws.t0; // (no exit: what the walk record keeps beside its end mark)
-    ++ws.n;
-    if (ws.n > max_steps || ws.beg > ws.end || ws.end > sc.num_adj) {
-        ws.alive = false;
-        return;
-    }
-    const uint32_t nf = ws.end - ws.beg;
-    const float t0 = ws.t0;
-    float t1 = __builtin_bit_cast(float, 0x7f800000u);
-    float tmin_u = t1;
-    bool below = false;
-    uint32_t best = kNoIndex, bw = kDeltaNone;
-    float t1m = t1;
-    const float t0m = t0 * (1.0f - 0x1p-21f);
-    const float t0p = t0 * (1.0f + 0x1p-21f);
-    const uint2 *__restrict__ row = sc.diff + ws.beg;
-    for (uint32_t k0 = 0; k0 < nf; k0 += G * U) {
-        if (k0 != 0) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) h[u] = row[k0 + u * G + sub];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t k = k0 + u * G + sub;
-            const float dx = f16_to_f32(h[u].x);
-            const float dy = f16_to_f32(h[u].x >> 16);
-            const float dz = f16_to_f32(h[u].y);
-            const float fx = fmaf(dx, 0.5f, ws.xc[0]);
-            const float fy = fmaf(dy, 0.5f, ws.xc[1]);
-            const float fz = fmaf(dz, 0.5f, ws.xc[2]);
-            const float dp = sdf_dot3(dx, dy, dz, ray.dx, ray.dy, ray.dz);
-            const float num = sdf_dot3(fx - ray.ox, fy - ray.oy, fz - ray.oz, dx, dy, dz);
-            const bool pos = dp > 0.0f && k < nf;
-            // the division filter of walk_advance
-            const float lo = fmaf(t0m, dp, -0x1p-126f);
-            bool maybe = pos && num < fmaf(t1m, dp, 0x1p-126f) && num > lo;
-            if constexpr (DUAL) {
-                below = below || (pos && num < lo);
-                maybe = maybe || (pos && num >= lo && num <= fmaf(t0p, dp, 0x1p-126f));
-            }
-            if (maybe) {
-                const float t = num / dp;
-                if (t > t0 && t < t1) {
-                    t1 = t;
-                    t1m = fmaf(fabsf(t), 0x1p-21f, t);
-                    best = k;
-                    bw = h[u].y >> 16;
-                }
-                if constexpr (DUAL) tmin_u = fminf(tmin_u, t);
-            }
-        }
-    }
-    // the first minimum in row order: the smallest t, then the smallest k
-    uint32_t bl = below ? 1u : 0u;
-#pragma unroll
-    for (int s = 0; (1 << s) < G; ++s) {
-        const float ot = __builtin_bit_cast(float, split_xor<G>(__builtin_bit_cast(uint32_t, t1), s));
-        const uint32_t ob = split_xor<G>(best, s), ow = split_xor<G>(bw, s);
-        const bool take = ot < t1 || (ot == t1 && ob < best);
-        t1 = take ? ot : t1;
-        best = take ? ob : best;
-        bw = take ? ow : bw;
-        if constexpr (DUAL) {
-            bl |= split_xor<G>(bl, s);
-            tmin_u = fminf(tmin_u, __builtin_bit_cast(float, split_xor<G>(
-                                       __builtin_bit_cast(uint32_t, tmin_u), s)));
-        }
-    }
-    if constexpr (DUAL) si.agrees = !(bl != 0u || tmin_u <= t0);
-    if (best == kNoIndex) {
-        ws.alive = false;
-        return;
-    }
-    const uint32_t next = bw != kDeltaNone
-                              ? (uint32_t)((int32_t)ws.cell + (int32_t)(int16_t)(uint16_t)bw)
-                              : sc.adj[ws.beg + best];
-    if (next >= sc.num_points) {
-        ws.alive = false;
-        return;
-    }
-    si.found = true;
-    si.next = next;
-    si.t1 = t1;
-    load_cell<RB>(sc, next, si.xn, si.beg, si.end);
-    si.stepped = t1 > t0;
-}
-
 // slots of the block's contribution table: one per step between flushes
 constexpr uint32_t kSplitSlots = 64u * kChunkTrips;
 
@@ -1199,14 +1045,6 @@ struct BackwardLane {
     bool valid;
 };
 
-// First wavefront of block b: tiles (4 G wavefronts, G blocks) go round robin
-// over the XCDs.
-template <int G>
-__device__ __forceinline__ uint32_t split_wave(uint32_t b) {
-    const uint32_t x = b % kXcds, k = b / kXcds;
-    return (((k / G) * kXcds + x) * G + k % G) * 4u;
-}
-
 template <int G>
 __device__ __forceinline__ BackwardLane backward_lane(const BwdArgs &a) {
     BackwardLane b;
@@ -1725,7 +1563,7 @@ static inline dim3 grid_for(uint64_t n) { return dim3((unsigned)((n + kBlock - 1
 //   900k / 30k       1.14/1.40  1.44/1.54     1.84/2.41
 // (two lanes shorten the backward even where the chip is full: 32 rays over six
 // trips meet fewer distinct cells than 64 rays over three).
-static int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered) {
+int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered) {
     if (num_rays < 2ull * num_points) {
         if (num_rays <= 16384u) return 16;
         if (num_rays <= 49152u) return 8;
@@ -1820,14 +1658,15 @@ hipError_t launch_record_reset(const WalkRecordArgs &r, uint64_t table_words, hi
 // before offs[0], the last one those from offs[N] up to num_adj and the
 // table's zero padding, as prefetch_diff_kernel does.  Record words past the
 // attribute row are left unwritten (nothing reads them).  The offset table
-// built with the cell table carries each entry's neighbour in its fourth
-// half (`neighbour_delta`), so the walk over the cell table reads the exit
+// built with the cell table (from the points, or from a caller's table:
+// `given`) carries each entry's neighbour in its fourth half (`neighbour_delta`), so the walk over the cell table reads the exit
 // face's neighbour from the entry it already holds.  CELLS = false: the
 // offset table alone, as prefetch_adjacent_diff gives it (fourth half 0).
 template <int L, typename AT, bool CELLS = true>
 __global__ __launch_bounds__(kBlock) void scene_prep_kernel(const SceneView sc, uint32_t *cells,
                                                             uint2 *diff, AT *contribution,
-                                                            float *alpha) {
+                                                            float *alpha,
+                                                            const uint2 *__restrict__ given) {
     constexpr uint32_t D = 1 + 3 * (L + 1) * (L + 1);
     constexpr uint32_t RW = cell_record_bytes(L, sizeof(AT)) / 4;
     constexpr uint32_t A = kCellAttrByte / 4;
@@ -1893,7 +1732,10 @@ __global__ __launch_bounds__(kBlock) void scene_prep_kernel(const SceneView sc, 
             // with the cell table, the entry's fourth half (0 in the plain
             // table) holds the neighbour relative to the row's cell
             const uint32_t w = CELLS ? neighbour_delta(c0 + row, a) : 0u;
-            if (a >= sc.num_points) {
+            if (CELLS && given) {
+                const uint2 g = given[k];
+                diff[k] = make_uint2(g.x, (g.y & 0xffffu) | (w << 16));
+            } else if (a >= sc.num_points) {
                 diff[k] = make_uint2(0x7e007e00u, 0x7e00u | (w << 16)); // NaN plane
             } else {
                 const float qx = sc.points[3ull * a], qy = sc.points[3ull * a + 1],
@@ -1922,31 +1764,34 @@ hipError_t launch_prefetch_diff(const float *points, uint32_t num_points, uint32
     sc.num_adj = num_adj;
     const uint32_t waves = (num_points + 63u) / 64u;
     hipLaunchKernelGGL((scene_prep_kernel<0, float, false>), dim3((waves + kBlock / 64 - 1) / (kBlock / 64)),
-                       dim3(kBlock), 0, stream, sc, nullptr, diff, nullptr, nullptr);
+                       dim3(kBlock), 0, stream, sc, nullptr, diff, nullptr, nullptr,
+                       nullptr);
     return hipGetLastError();
 }
 
 template <typename AT>
 static hipError_t launch_scene_prep_T(int L, const SceneView &sc, uint32_t *cells, uint2 *diff,
-                                      void *contribution, float *alpha, hipStream_t stream) {
+                                      void *contribution, float *alpha, const uint2 *given,
+                                      hipStream_t stream) {
     AT *co = static_cast<AT *>(contribution);
     const uint32_t waves = (sc.num_points + 63u) / 64u;
     const dim3 grid((waves + kBlock / 64 - 1) / (kBlock / 64));
     switch (L) {
-    case 0: hipLaunchKernelGGL((scene_prep_kernel<0, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha); break;
-    case 1: hipLaunchKernelGGL((scene_prep_kernel<1, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha); break;
-    case 2: hipLaunchKernelGGL((scene_prep_kernel<2, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha); break;
-    case 3: hipLaunchKernelGGL((scene_prep_kernel<3, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha); break;
+    case 0: hipLaunchKernelGGL((scene_prep_kernel<0, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha, given); break;
+    case 1: hipLaunchKernelGGL((scene_prep_kernel<1, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha, given); break;
+    case 2: hipLaunchKernelGGL((scene_prep_kernel<2, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha, given); break;
+    case 3: hipLaunchKernelGGL((scene_prep_kernel<3, AT>), grid, dim3(kBlock), 0, stream, sc, cells, diff, co, alpha, given); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_scene_prep(int L, bool half, const SceneView &sc, uint32_t *cells, uint2 *diff,
-                             void *contribution, float *alpha, hipStream_t stream) {
+                             void *contribution, float *alpha, const uint2 *given,
+                             hipStream_t stream) {
     if (sc.num_points == 0) return hipSuccess;
-    return half ? launch_scene_prep_T<_Float16>(L, sc, cells, diff, contribution, alpha, stream)
-                : launch_scene_prep_T<float>(L, sc, cells, diff, contribution, alpha, stream);
+    return half ? launch_scene_prep_T<_Float16>(L, sc, cells, diff, contribution, alpha, given, stream)
+                : launch_scene_prep_T<float>(L, sc, cells, diff, contribution, alpha, given, stream);
 }
 
 template <typename AT>
@@ -2162,135 +2007,6 @@ hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, 
         return hipErrorInvalidValue;
     }
 #undef SDF_FINALIZE
-}
-
-// ---------------------------------------------------------------------------
-// inference render (the reference's `benchmark` kernel,
-// src/tracing/pipeline.cu:1067-1199)
-
-// One lane per pixel, 16x16 pixel tiles per block as the traced kernels.  The
-// step is the forward's compositing without its per-point outputs; the walk
-// reads the caller's unpadded offset table with guarded loads.
-template <int L, bool NEUS, typename AT>
-__global__ __launch_bounds__(kBlock) void render_kernel(RenderArgs a) {
-    constexpr int nsh = (L + 1) * (L + 1);
-    constexpr int D = 1 + 3 * nsh;
-    __shared__ float sh_all[kBlock * nsh];
-    bool valid;
-    const uint32_t px = ray_for_lane<kForwardChunk>(a.width * a.height, a.width, a.num_tiles, valid);
-    const uint32_t pi = valid ? px % a.width : 0u, pj = valid ? px / a.width : 0u;
-
-    RayF ray = {};
-    bool masked = false;
-    if (valid) {
-        float dir[3];
-        sdf_cast_ray(a.forward, a.right, a.up, a.fov, a.focal, a.width, a.height, a.model, pi,
-                     pj, dir);
-        const float n = sqrtf(sdf_dot3(dir[0], dir[1], dir[2], dir[0], dir[1], dir[2]));
-        masked = n < 0.1f;
-        ray.ox = a.position[0];
-        ray.oy = a.position[1];
-        ray.oz = a.position[2];
-        if (!masked) {
-            // ray.direction /= ray.direction.norm()
-            ray.dx = dir[0] / n;
-            ray.dy = dir[1] / n;
-            ray.dz = dir[2] / n;
-        }
-    }
-    float *sh = sh_all + threadIdx.x; // basis function k at sh[k * kBlock]
-    {
-        float sh0[nsh];
-        sh_basis<L>(ray.dx, ray.dy, ray.dz, sh0);
-#pragma unroll
-        for (int k = 0; k < nsh; ++k) sh[k * kBlock] = sh0[k];
-    }
-    const float sha = a.sharpness[0];
-    const int32_t sdf_ch = a.settings.sdf_channel;
-    const bool neus_alpha = NEUS && sdf_ch >= 0;
-    const float thr = a.settings.weight_threshold;
-
-    float T = 1.0f;
-    float C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
-    WalkState ws;
-    walk_init(a.scene, (valid && !masked) ? a.start[0] : kNoIndex, ws);
-    WalkCounters wc = {0u, 0u, 0ull, 0ull};
-
-    while (__ballot(ws.alive) != 0ull) {
-        StepInfo si;
-        si.stepped = false;
-        si.found = false;
-        if (ws.alive)
-            walk_advance<true, false, true>(a.scene, ray, a.settings.max_intersections, ws, si,
-                                            wc);
-        bool keep = true;
-        if (si.stepped) {
-            const AT *__restrict__ row = static_cast<const AT *>(a.scene.attrs) + (uint64_t)ws.cell * D;
-            float s = (float)row[D - 1];
-            const float dt = fmaxf(si.t1 - ws.t0, 0.0f);
-            if (neus_alpha) {
-                const float d = (float)row[sdf_ch];
-                const float phi = sdf_sigmoidf(-sha * d);
-                s = sha * phi * (1.0f - phi);
-            }
-            const float alpha = 1.0f - sdf_expf(-s * dt);
-            const float w = T * alpha;
-            float r, g, b;
-            if (NEUS || (float)row[D - 1] > 1e-6f) {
-                sh_rgb<L>(sh, kBlock, row, r, g, b);
-            } else {
-                r = g = b = 0.0f;
-            }
-            C0 = fmaf(w, r, C0);
-            C1 = fmaf(w, g, C1);
-            C2 = fmaf(w, b, C2);
-            T = T * (1.0f - alpha);
-            keep = T > thr;
-        }
-        if (si.stepped && !keep) ws.alive = false;
-        if (ws.alive && si.found) walk_move(ws, si);
-    }
-
-    if (!valid) return;
-    const uint64_t out_idx = (uint64_t)(a.height - 1u - pj) * a.width + pi;
-    if (masked) {
-        a.out[out_idx] = sdf_make_rgba8(a.bg[0], a.bg[1], a.bg[2], 1.0f);
-        return;
-    }
-    float bg0 = a.bg[0], bg1 = a.bg[1], bg2 = a.bg[2];
-    if (a.checker_bg) {
-        const int is = 2 * (int)((pi / 20u) % 2u) - 1;
-        const int js = 2 * (int)((pj / 20u) % 2u) - 1;
-        bg0 = bg1 = bg2 = (is * js > 0) ? 0.3f : 0.5f;
-    }
-    a.out[out_idx] = sdf_make_rgba8(fmaf(T, bg0, C0), fmaf(T, bg1, C1), fmaf(T, bg2, C2), 1.0f);
-}
-
-template <int L, typename AT>
-static hipError_t launch_render_L(const RenderArgs &a, bool neus, hipStream_t stream) {
-    const dim3 grid(grid_blocks_for_tiles(a.num_tiles));
-    if (neus) {
-        hipLaunchKernelGGL((render_kernel<L, true, AT>), grid, dim3(kBlock), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((render_kernel<L, false, AT>), grid, dim3(kBlock), 0, stream, a);
-    }
-    return hipGetLastError();
-}
-
-template <typename AT>
-static hipError_t launch_render_T(int L, const RenderArgs &a, bool neus, hipStream_t stream) {
-    switch (L) {
-    case 0: return launch_render_L<0, AT>(a, neus, stream);
-    case 1: return launch_render_L<1, AT>(a, neus, stream);
-    case 2: return launch_render_L<2, AT>(a, neus, stream);
-    case 3: return launch_render_L<3, AT>(a, neus, stream);
-    default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_render(int L, const RenderArgs &a, bool neus, bool half, hipStream_t stream) {
-    return half ? launch_render_T<_Float16>(L, a, neus, stream)
-                : launch_render_T<float>(L, a, neus, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -793,11 +793,18 @@ class Pipeline:
         vis.checker_bg = 1 if checker_bg else 0
         dev = output_rgba.device
         with torch.cuda.device(dev):
-            check(_lib.lib().sdf_trace_benchmark(
+            L = _lib.lib()
+            nbytes = int(L.sdf_trace_benchmark_scratch_bytes(
+                self._sh_degree, settings.attr_type, num_points, num_adj, cam.width, cam.height))
+            base = None
+            if nbytes:
+                scratch = torch.empty(nbytes + 256, dtype=torch.uint8, device=dev)
+                base = (scratch.data_ptr() + 255) & ~255
+            check(L.sdf_trace_benchmark_planned(
                 self._sh_degree, C.byref(settings), num_points, ptr(points_c),
                 ptr(attributes_c), num_adj, ptr(adj_c), ptr(offs_c), ptr(diff_c),
                 diff_c.numel() // 4, C.byref(cam), C.byref(vis), ptr(start_point),
-                ptr(output_rgba), ptr(sharpness), _lib.stream_handle(dev)))
+                ptr(output_rgba), ptr(sharpness), base, nbytes, _lib.stream_handle(dev)))
 
     # -- walk statistics (measurement / parity hook) -------------------------
     def walk_stats(self, points, attributes, point_adjacency, point_adjacency_offsets, rays,

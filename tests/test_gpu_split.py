@@ -91,3 +91,51 @@ def test_split_backward(torch_dev, oracle_lib, cfg, shape, mode):
     _check_backward(bwd, st, ref, w)
     bwd, st, ref = _backward_both(w, torch_dev, oracle_lib, mode)  # scanning
     _check_backward(bwd, st, ref, w)
+
+
+# one pixel (the caller's arrays), then 16, 4, 2 lanes and one over C1, 8 and 4 over C2
+@pytest.mark.parametrize("mode,dtype", [("sdfoam", "float32"), ("standard", "float16")])
+@pytest.mark.parametrize("cfg,width,height", [
+    (1, 1, 1), (1, 9, 7), (1, 64, 64), (1, 91, 91), (1, 257, 255), (1, 300, 301), (1, 500, 501),
+    (2, 131, 127), (2, 300, 301),
+])
+def test_split_render_same_image(torch_dev, cfg, width, height, mode, dtype):
+    """The render over the frame's tables equals the one over the caller's
+    arrays (sdf_trace_benchmark), pixel for pixel."""
+    import ctypes as C
+
+    import torch
+
+    import sdfoam_amd
+    from sdfoam_amd import _lib, scenes
+
+    w = scene(cfg, mode=mode)
+    g = gpu_scene(w, torch_dev)
+    g["attributes"] = g["attributes"].to(getattr(torch, dtype))
+    scene_args = [g[k] for k in ("points", "attributes", "point_adjacency",
+                                 "point_adjacency_offsets")]
+    diff = sdfoam_amd.prefetch_adjacent_diff(*(scene_args[i] for i in (0, 2, 3)))
+    diff = diff[: scene_args[2].numel()].clone()
+    diff[:, 3] = 7.0  # the fourth column is the caller's: not read
+    pipe = sdfoam_amd.create_pipeline(w.sh_degree, dtype)
+    cam = scenes.camera_dict(w.extra["camera"], width=width, height=height)
+    start = g["start_point"].view(torch.int32).reshape(-1)[:1].clone().view(torch.uint32)
+    inv = torch.tensor([w.inv_s], device=torch_dev)
+    got = torch.zeros((height, width), dtype=torch.int32, device=torch_dev).view(torch.uint32)
+    pipe.trace_benchmark(*scene_args, diff, cam, start, got, weight_threshold=1e-3,
+                         alpha_mode=mode, inv_s=inv)
+    want = torch.zeros_like(got.view(torch.int32))
+    c = _lib.Camera()
+    for key in ("position", "forward", "up", "right"):
+        getattr(c, key)[:] = [float(x) for x in cam[key]]
+    c.fov, c.width, c.height, c.model = cam["fov"], width, height, _lib.SDF_CAMERA_PINHOLE
+    vis = _lib.Visualization()
+    vis.bg_color[:] = [1.0, 1.0, 1.0]
+    settings = pipe._settings(1e-3, None, mode, None)
+    p = [t.data_ptr() for t in scene_args]
+    _lib.check(_lib.lib().sdf_trace_benchmark(
+        w.sh_degree, C.byref(settings), w.num_points, p[0], p[1], scene_args[2].numel(), p[2], p[3],
+        diff.data_ptr(), diff.shape[0], C.byref(c), C.byref(vis), start.data_ptr(),
+        want.data_ptr(), inv.data_ptr(), _lib.stream_handle(torch_dev)))
+    assert torch.equal(got.view(torch.int32), want)
+    assert len(torch.unique(want)) > 1 or width == 1
