@@ -455,17 +455,15 @@ SDF_HD uint32_t sphere_columns(const Sphere &S) {
 // sphere must be decided.
 constexpr uint32_t kStatusClean = 4u;
 
-// Points of column `col` against the sphere: 0 if one lies strictly inside,
-// 2 if none does but one's sign is undecided and it is certified or clean (an
-// open point exactly on the sphere is passed over: the candidates' own
-// triangulation of the open points already chose among such points), 1
-// otherwise.
-SDF_HD uint32_t sphere_scan_column(const float *p, const uint32_t *v, const GridView &gv,
-                                   const uint32_t *status, const Sphere &S, uint32_t col) {
+// The cells x0 .. x1 (none where x0 > x1) of column `col` that the sphere may
+// reach, and the column's y and z.
+SDF_HD void sphere_column_cells(const GridView &gv, const Sphere &S, uint32_t col, int &x0,
+                                int &x1, int &cy, int &cz) {
     const GridGeom &g = gv.g;
     const GridLevel &lv = g.level[S.l];
     const uint32_t ny = (uint32_t)(S.hi_c[1] - S.lo_c[1] + 1);
-    const int cy = S.lo_c[1] + (int)(col % ny), cz = S.lo_c[2] + (int)(col / ny);
+    cy = S.lo_c[1] + (int)(col % ny);
+    cz = S.lo_c[2] + (int)(col / ny);
     // squared distance from the centre to the column's y and z extent
     double rem = S.r * S.r;
     const int cc[3] = {0, cy, cz};
@@ -476,26 +474,48 @@ SDF_HD uint32_t sphere_scan_column(const float *p, const uint32_t *v, const Grid
             S.ctr[k] < blo ? blo - S.ctr[k] : (S.ctr[k] > bhi ? S.ctr[k] - bhi : 0.0);
         rem -= e * e;
     }
-    if (rem < 0.0) return 1u;
+    x0 = 1;
+    x1 = 0;
+    if (rem < 0.0) return;
     const double w = sqrt(rem);
-    const int x0 = axis_cell(S.o[0] + S.ctr[0] - w - g.slack, g.lo[0], lv.inv_h, lv.dims[0]);
-    const int x1 = axis_cell(S.o[0] + S.ctr[0] + w + g.slack, g.lo[0], lv.inv_h, lv.dims[0]);
-    const uint32_t *sorted = gv.sorted[S.l];
+    x0 = axis_cell(S.o[0] + S.ctr[0] - w - g.slack, g.lo[0], lv.inv_h, lv.dims[0]);
+    x1 = axis_cell(S.o[0] + S.ctr[0] + w + g.slack, g.lo[0], lv.inv_h, lv.dims[0]);
+    x0 = x0 > S.lo_c[0] ? x0 : S.lo_c[0];
+    x1 = x1 < S.hi_c[0] ? x1 : S.hi_c[0];
+}
+
+// Point k of the grid's order against the sphere: 0 strictly inside, 2 its
+// sign is undecided and it is certified or clean (an open point exactly on
+// the sphere is passed over: the candidates' own triangulation of the open
+// points already chose among such points), 1 otherwise.
+SDF_HD uint32_t sphere_test_point(const uint32_t *v, const GridView &gv, const uint32_t *status,
+                                  const Sphere &S, uint32_t k) {
+    const uint32_t j = gv.sorted[S.l][k];
+    if (j == v[0] || j == v[1] || j == v[2] || j == v[3]) return 1u;
+    const float *sp = gv.spts + 4ull * k;
+    double q[3];
+    for (int m = 0; m < 3; ++m) q[m] = (double)sp[m] - S.o[m];
+    const double e0 = q[0] - S.ctr[0], e1 = q[1] - S.ctr[1], e2 = q[2] - S.ctr[2];
+    if (e0 * e0 + e1 * e1 + e2 * e2 > S.r * S.r) return 1u; // clearly outside
+    const int s = vcell::in_sphere(S.pl[0].n, S.pl[1].n, S.pl[2].n, q);
+    if (s > 0) return 0u;
+    return s == 0 && (status[j] == vcell::kCertified || status[j] == kStatusClean) ? 2u : 1u;
+}
+
+// The points of column `col`: 0 if one lies strictly inside the sphere, 2 if
+// none does but one is undecided (sphere_test_point), 1 otherwise.
+SDF_HD uint32_t sphere_scan_column(const uint32_t *v, const GridView &gv, const uint32_t *status,
+                                   const Sphere &S, uint32_t col) {
+    int x0, x1, cy, cz;
+    sphere_column_cells(gv, S, col, x0, x1, cy, cz);
     uint32_t res = 1u;
-    for (int cx = x0 > S.lo_c[0] ? x0 : S.lo_c[0]; cx <= (x1 < S.hi_c[0] ? x1 : S.hi_c[0]); ++cx) {
+    for (int cx = x0; cx <= x1; ++cx) {
         uint32_t begin, end;
         cell_range_grouped(gv, S.l, (uint32_t)cx, (uint32_t)cy, (uint32_t)cz, begin, end);
         for (uint32_t k = begin; k < end; ++k) {
-            const uint32_t j = sorted[k];
-            if (j == v[0] || j == v[1] || j == v[2] || j == v[3]) continue;
-            const float *sp = gv.spts + 4ull * k;
-            double q[3];
-            for (int m = 0; m < 3; ++m) q[m] = (double)sp[m] - S.o[m];
-            const double e0 = q[0] - S.ctr[0], e1 = q[1] - S.ctr[1], e2 = q[2] - S.ctr[2];
-            if (e0 * e0 + e1 * e1 + e2 * e2 > S.r * S.r) continue; // clearly outside
-            const int s = vcell::in_sphere(S.pl[0].n, S.pl[1].n, S.pl[2].n, q);
-            if (s > 0) return 0u;
-            if (s == 0 && (status[j] == vcell::kCertified || status[j] == kStatusClean)) res = 2u;
+            const uint32_t r = sphere_test_point(v, gv, status, S, k);
+            if (r == 0u) return 0u;
+            if (r == 2u) res = 2u;
         }
     }
     return res;
@@ -511,7 +531,7 @@ SDF_HD uint32_t sphere_empty(const float *p, const uint32_t *v, const GridView &
     uint32_t res = 1u;
     const uint32_t cols = sphere_columns(S);
     for (uint32_t c = 0; c < cols; ++c) {
-        const uint32_t r = sphere_scan_column(p, v, gv, status, S, c);
+        const uint32_t r = sphere_scan_column(v, gv, status, S, c);
         if (r == 0u) return 0u;
         if (r == 2u) res = 2u;
     }
