@@ -262,10 +262,13 @@ struct StagedVert {
     double x[3], e, r2;
 };
 
-// A cell vertex as the batch test reads it (position and error bound).
+// A cell vertex as the batch test reads it: its position, and its error bound
+// with the test's rounding per unit of |q| (4 eps max |x|).
 struct TestVert {
     double x[3], e;
 };
+
+constexpr uint32_t kBoundR2 = 0, kBoundErr = 1, kBoundLo = 2, kBoundHi = 5;
 
 struct WaveShared {
     double pn[kWavePlanes][3]; // plane normals
@@ -280,7 +283,9 @@ struct WaveShared {
         StagedVert stg[kWaveNew];     // wave_clip's new vertices
         TestVert tv[kWaveVerts];      // wave_may_cut's copy of the vertices
     };
-    double mr2, blo[3], bhi[3]; // max |v|^2 and the vertices' box (the cell's bounds)
+    // the cell's bounds: max |v|^2, the largest error bound, and the vertices'
+    // box (lower and upper corner)
+    double bound[8];
 };
 
 struct WaveCell {
@@ -323,27 +328,39 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
     return __builtin_bit_cast(double, (uint64_t)readlane_u((uint32_t)(b >> 32), lane) << 32 |
                                           readlane_u((uint32_t)b, lane));
 }
-// Maximum / minimum over the wave (every lane active): lane 15 of each row
-// gathers its row by shifts of 1, 2, 4 and 8 (a lane without a source keeps
-// its own value, which max and min ignore), rows 1 and 3 take rows 0 and 2,
-// rows 2 and 3 take lane 31, and lane 63 holds the result.
-__device__ __forceinline__ double wmaxd(double v) {
-    v = fmax(v, dpp_d<0x111>(v));
-    v = fmax(v, dpp_d<0x112>(v));
-    v = fmax(v, dpp_d<0x114>(v));
-    v = fmax(v, dpp_d<0x118>(v));
-    v = fmax(v, dpp_d<0x142, 0xa>(v));
-    v = fmax(v, dpp_d<0x143, 0xc>(v));
-    return readlane_d(v, 63);
+// The same for moves in which every lane has a source (row_ror:k = 0x120 + k):
+// no copy of the old value is needed.
+template <int CTRL> __device__ __forceinline__ double dpp_ror_d(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo);
 }
-__device__ __forceinline__ double wmind(double v) {
-    v = fmin(v, dpp_d<0x111>(v));
-    v = fmin(v, dpp_d<0x112>(v));
-    v = fmin(v, dpp_d<0x114>(v));
-    v = fmin(v, dpp_d<0x118>(v));
-    v = fmin(v, dpp_d<0x142, 0xa>(v));
-    v = fmin(v, dpp_d<0x143, 0xc>(v));
-    return readlane_d(v, 63);
+// maximum over the four rows' lanes of one index (v_permlane16_swap and
+// v_permlane32_swap exchange rows between two registers)
+__device__ __forceinline__ double rows_max(double v) {
+    uint64_t b = __builtin_bit_cast(uint64_t, v);
+    auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    v = fmax(__builtin_bit_cast(double, (uint64_t)h16[0] << 32 | l16[0]),
+             __builtin_bit_cast(double, (uint64_t)h16[1] << 32 | l16[1]));
+    b = __builtin_bit_cast(uint64_t, v);
+    auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    return fmax(__builtin_bit_cast(double, (uint64_t)h32[0] << 32 | l32[0]),
+                __builtin_bit_cast(double, (uint64_t)h32[1] << 32 | l32[1]));
+}
+// Minimum over the wave (every lane active): each row gathers its 16 lanes by
+// rotations of 1, 2, 4 and 8, rows 1 and 3 take rows 0 and 2, rows 2 and 3
+// take lane 31, and lane 63 holds the result.
+__device__ __forceinline__ uint32_t wminu(uint32_t v) {
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x121, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x122, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, false));
+    v = min(v, dpp_u<0x142, 0xa>(~0u, v));
+    v = min(v, dpp_u<0x143, 0xc>(~0u, v));
+    return readlane_u(v, 63);
 }
 // inclusive prefix maximum over the lanes (every lane active), as wscanu
 __device__ __forceinline__ uint32_t wscanmaxu(uint32_t v) {
@@ -387,30 +404,38 @@ __device__ __forceinline__ uint32_t range_owner(uint8_t *owner, uint32_t cnt, ui
 
 __device__ __forceinline__ uint32_t plane_of(uint32_t vp, int k) { return (vp >> (8 * k)) & 0xffu; }
 
+// Of two values per lane, each lane keeps the maximum over itself and its
+// partner of one: the odd lanes' second, the others' first.
+template <int CTRL> __device__ __forceinline__ double split_max(double a, double b, bool odd) {
+    return fmax(odd ? b : a, dpp_ror_d<CTRL>(odd ? a : b));
+}
+
 // max |v|^2 and the vertices' box grown by the largest error bound
-// (dgrid::vertex_box).
+// (dgrid::vertex_box).  The eight maxima over the wave are halved and shared
+// out: lane ^ 1 keeps four of them, lane ^ 2 two, and lane l ends with value
+// l & 7, in 12 maxima instead of eight reductions of six each.
 __device__ void wave_bounds(WaveCell &c, WaveShared &sh) {
-    double r2 = 0.0, e = 0.0, lo[3], hi[3];
-    for (int k = 0; k < 3; ++k) {
-        lo[k] = INFINITY;
-        hi[k] = -INFINITY;
-    }
+    const uint32_t l = wlane();
+    double v[8] = {0.0, 0.0};
+    for (int k = 2; k < 8; ++k) v[k] = -INFINITY;
     for (int s = 0; s < 2; ++s) {
         if (c.vp[s] == kFree) continue;
-        r2 = fmax(r2, c.vr2[s]);
-        e = fmax(e, c.ve[s]);
+        v[kBoundR2] = fmax(v[kBoundR2], c.vr2[s]);
+        v[kBoundErr] = fmax(v[kBoundErr], c.ve[s]);
         for (int k = 0; k < 3; ++k) {
-            lo[k] = fmin(lo[k], c.vx[s][k]);
-            hi[k] = fmax(hi[k], c.vx[s][k]);
+            v[kBoundLo + k] = fmax(v[kBoundLo + k], -c.vx[s][k]);
+            v[kBoundHi + k] = fmax(v[kBoundHi + k], c.vx[s][k]);
         }
     }
-    // every lane stores the same values; the wave's own later reads see them
-    sh.mr2 = wmaxd(r2);
-    e = wmaxd(e);
-    for (int k = 0; k < 3; ++k) {
-        sh.blo[k] = wmind(lo[k]) - e;
-        sh.bhi[k] = wmaxd(hi[k]) + e;
-    }
+    for (int k = 0; k < 4; ++k) v[k] = split_max<0xb1>(v[2 * k], v[2 * k + 1], l & 1u);
+    for (int k = 0; k < 2; ++k) v[k] = split_max<0x4e>(v[2 * k], v[2 * k + 1], l & 2u);
+    double x = split_max<0x124>(v[0], v[1], l & 4u);
+    x = fmax(x, dpp_ror_d<0x128>(x));
+    x = rows_max(x);
+    const double e = readlane_d(x, kBoundErr);
+    if (l >= kBoundLo) x += e;
+    if (l < 8u) sh.bound[l] = l >= kBoundLo && l < kBoundHi ? -x : x;
+    __syncthreads();
 }
 
 __device__ void wave_init(WaveCell &c, WaveShared &sh, const double *rlo, const double *rhi) {
@@ -637,9 +662,12 @@ __device__ int wave_clip(WaveCell &c, WaveShared &sh, const double *q, double qc
 // The lanes whose candidate plane (relative position q, qc = |q|^2 / 2;
 // `mine`: the lane holds one) may cut the cell: each lane tests its plane
 // against every vertex (copied to LDS), and a plane that leaves every
-// vertex inside by more than the bound wave_clip uses (the vertex's error
-// bound and the dot product's rounding) misses the cell, and every cell the
-// clips that follow make (they only shrink it).  One pass for a batch of
+// vertex inside by more than a bound on the vertex's error and the test's
+// rounding misses the cell, and every cell the clips that follow make (they
+// only shrink it).  Three fused steps round x.q - qc by at most 3 eps (|x.q|'s
+// terms + qc) <= 3 eps (max |x| |q|_1 + qc); the bound takes 4 eps of it, so a
+// vertex takes four fused operations and a compare instead of twelve
+// operations.  One pass for a batch of
 // candidates in place of a wave_clip call each, most of which find no cut
 // where the cell is large.
 __device__ uint64_t wave_may_cut(const WaveCell &c, WaveShared &sh, bool mine, const double *q,
@@ -652,20 +680,19 @@ __device__ uint64_t wave_may_cut(const WaveCell &c, WaveShared &sh, bool mine, c
         t.x[0] = c.vx[s][0];
         t.x[1] = c.vx[s][1];
         t.x[2] = c.vx[s][2];
-        t.e = c.ve[s];
+        t.e = c.ve[s] + 4.0 * vcell::kEps *
+                            fmax(fmax(vcell::dabs(t.x[0]), vcell::dabs(t.x[1])),
+                                 vcell::dabs(t.x[2]));
     }
     __syncthreads();
     bool cut = false;
     if (mine) {
         const double qn = vcell::dabs(q[0]) + vcell::dabs(q[1]) + vcell::dabs(q[2]);
+        const double cb = 4.0 * vcell::kEps * qc;
         for (uint32_t v = 0; v < nv && !cut; ++v) {
             const double *x = sh.tv[v].x;
-            const double sd = x[0] * q[0] + x[1] * q[1] + x[2] * q[2] - qc;
-            const double bound =
-                sh.tv[v].e * qn + 4.0 * vcell::kEps *
-                                      (vcell::dabs(x[0] * q[0]) + vcell::dabs(x[1] * q[1]) +
-                                       vcell::dabs(x[2] * q[2]) + qc);
-            cut = !(sd < -bound);
+            const double sd = fma(x[0], q[0], fma(x[1], q[1], fma(x[2], q[2], -qc)));
+            cut = !(sd < -fma(sh.tv[v].e, qn, cb));
         }
     }
     const uint64_t m = wballot(cut);
@@ -718,12 +745,26 @@ __device__ bool wave_touches_box(const WaveCell &c, const WaveShared &sh) {
     return wballot(t) != 0ull;
 }
 
+// The point of block b of a launch of `blocks`, in the grid's Morton order
+// (or the query's): the XCDs take turns on runs of kCertifyRun points, so that
+// neighbouring cells are looked up and their points read through one L2 (the
+// caller's order leaves neighbours on all of them; runs of 16 take as long).
+constexpr uint32_t kCertifyRun = 64;
+
+__device__ __forceinline__ uint32_t certify_slot(uint32_t b, uint32_t blocks) {
+    const uint32_t full = blocks / (kXcds * kCertifyRun) * (kXcds * kCertifyRun);
+    const uint32_t k = b / kXcds, x = b % kXcds;
+    return b < full ? ((k / kCertifyRun) * kXcds + x) * kCertifyRun + k % kCertifyRun : b;
+}
+
 // counters: 0 report rows asked for, 1 open points, 2 undecided cells,
 // 3 cells over the fixed capacity, 4 coincident point pairs seen (twice).
-// One 64-thread block per point (per entry of `query` when it is given).  Four waves per SIMD (128 VGPRs, 200 bytes
-// of spills per lane) run it ~20% faster than the two its natural register
-// count (203) allows; three (168 VGPRs, 40 bytes) run it ~10% slower than
-// four.  What is uniform over the wave and indexed at run time (the grid
+// One 64-thread block per point (per entry of `query` when it is given).
+// Bound by VALU issue (71% busy, ~13,000 instructions per cell): 1M points take
+// 30.4 ms, 39.4 before the points were taken in Morton order, |x| and the nearest
+// candidate cost one instruction per step, the bounds were shared out over the
+// lanes and the batch test took fused steps.  Four waves per SIMD (128 VGPRs, 32
+// bytes of spills per lane); two were ~20%, three ~10% slower on an earlier build.  What is uniform over the wave and indexed at run time (the grid
 // cell and searched rings per level) or needed by every lane (the cell's
 // bounds) lives in LDS, not in per-lane registers or scratch.
 template <bool EXHAUSTIVE>
@@ -740,7 +781,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
     // wave; indexed by level, so kept in LDS rather than scratch memory)
     __shared__ int hc[dgrid::kLevels][3];
     __shared__ int rings[dgrid::kLevels];
-    const uint32_t i = query ? query[blockIdx.x] : blockIdx.x;
+    const uint32_t slot = certify_slot(blockIdx.x, gridDim.x);
+    const uint32_t i = query ? query[slot] : gv.sorted[0][slot];
     if (i >= n) return;
     const uint32_t l = wlane();
     const GridGeom &g = gv.g;
@@ -827,10 +869,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
                             d2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2];
                             if (d2 == 0.0) {
                                 dup = true;
-                            } else if (d2 <= 4.0 * sh.mr2 * (1.0 + 1e-9)) {
+                            } else if (d2 <= 4.0 * sh.bound[kBoundR2] * (1.0 + 1e-9)) {
                                 double reach_q = 0.0, mag = d2;
                                 for (int m = 0; m < 3; ++m) {
-                                    const double bb = q[m] > 0.0 ? sh.bhi[m] : sh.blo[m];
+                                    const double bb = q[m] > 0.0 ? sh.bound[kBoundHi + m] : sh.bound[kBoundLo + m];
                                     reach_q += bb * q[m];
                                     mag += vcell::dabs(bb * q[m]);
                                 }
@@ -847,27 +889,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
                     }
                     uint64_t m = wballot(surv);
                     if (__popcll(m) >= kBatchTestMin) m = wave_may_cut(c, sh, surv, q, 0.5 * d2);
+                    // nearest first, by the distances as floats: the order only
+                    // decides how many of the clips cut
+                    const uint32_t near = __builtin_bit_cast(uint32_t, (float)d2);
                     bool clipped = false;
                     while (m) {
-                        // nearest first
                         const bool mine = (m >> l) & 1ull;
-                        const double dm = wmind(mine ? d2 : INFINITY);
-                        const uint64_t hit = wballot(mine && d2 == dm);
-                        const int src = __builtin_ctzll(hit);
+                        const uint32_t least = wminu(mine ? near : ~0u);
+                        const int src = __builtin_ctzll(wballot(mine && near == least));
                         m &= ~(1ull << src);
                         const double qq[3] = {readlane_d(q[0], src), readlane_d(q[1], src),
                                               readlane_d(q[2], src)};
                         const double dd = readlane_d(d2, src);
                         const int32_t jj = (int32_t)readlane_u(j, src);
-                        // the cell may have shrunk since the filter
-                        if (dd > 4.0 * sh.mr2 * (1.0 + 1e-9)) continue;
-                        double reach_q = 0.0, mag = dd;
-                        for (int mm = 0; mm < 3; ++mm) {
-                            const double bb = qq[mm] > 0.0 ? sh.bhi[mm] : sh.blo[mm];
-                            reach_q += bb * qq[mm];
-                            mag += vcell::dabs(bb * qq[mm]);
-                        }
-                        if (reach_q < 0.5 * dd - 1e-14 * mag) continue;
                         const int rc = wave_clip(c, sh, qq, 0.5 * dd, jj);
                         if (rc >= 2) {
                             st = rc == 2 ? vcell::kUncertain : vcell::kOverflow;
@@ -891,7 +925,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
             const double reach = (double)r * lv.h - g.slack;
             const double reach2 = all ? INFINITY : (reach > 0.0 ? reach * reach : 0.0);
             const bool box = wave_touches_box(c, sh);
-            if (4.0 * sh.mr2 * (1.0 + 1e-9) < reach2) {
+            if (4.0 * sh.bound[kBoundR2] * (1.0 + 1e-9) < reach2) {
                 st = box ? vcell::kOpen : vcell::kCertified;
                 decided = true;
                 break;
@@ -902,7 +936,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
                 break;
             }
             if (r >= dgrid::kMinRing &&
-                4.0 * sh.mr2 * (1.0 + 1e-9) > (dgrid::kMaxRing * lv.h) * (dgrid::kMaxRing * lv.h))
+                4.0 * sh.bound[kBoundR2] * (1.0 + 1e-9) > (dgrid::kMaxRing * lv.h) * (dgrid::kMaxRing * lv.h))
                 break;
         }
     }
@@ -929,10 +963,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
                 d2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2];
                 if (d2 == 0.0) {
                     dup = true;
-                } else if (d2 <= 4.0 * sh.mr2 * (1.0 + 1e-9)) {
+                } else if (d2 <= 4.0 * sh.bound[kBoundR2] * (1.0 + 1e-9)) {
                     double reach_q = 0.0, mag = d2;
                     for (int mm = 0; mm < 3; ++mm) {
-                        const double bb = q[mm] > 0.0 ? sh.bhi[mm] : sh.blo[mm];
+                        const double bb = q[mm] > 0.0 ? sh.bound[kBoundHi + mm] : sh.bound[kBoundLo + mm];
                         reach_q += bb * q[mm];
                         mag += vcell::dabs(bb * q[mm]);
                     }
@@ -947,12 +981,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ce
             }
             uint64_t m = wballot(surv);
             if (__popcll(m) >= kBatchTestMin) m = wave_may_cut(c, sh, surv, q, 0.5 * d2);
+            const uint32_t near = __builtin_bit_cast(uint32_t, (float)d2);
             bool clipped = false;
             while (m) {
                 const bool mine = (m >> l) & 1ull;
-                const double dm = wmind(mine ? d2 : INFINITY);
-                const uint64_t hit = wballot(mine && d2 == dm);
-                const int src = __builtin_ctzll(hit);
+                const uint32_t least = wminu(mine ? near : ~0u);
+                const int src = __builtin_ctzll(wballot(mine && near == least));
                 m &= ~(1ull << src);
                 const double qq[3] = {readlane_d(q[0], src), readlane_d(q[1], src),
                                       readlane_d(q[2], src)};

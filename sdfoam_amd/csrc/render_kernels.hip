@@ -12,7 +12,7 @@ namespace {
 // outputs.  CT: the walk reads a cell table and a padded copy of the caller's
 // offset table that names each face's neighbour, made for the frame
 // (scene_prep_kernel); else the caller's arrays, its unpadded table with
-// guarded loads.  RENDER_NOTE
+// guarded loads. 
 template <int L, bool NEUS, typename AT, int G, bool CT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT && G == 1 ? 6 : 1))) void render_kernel(RenderArgs a) {
     static_assert(G == 1 || CT, "lanes share a pixel over the cell table only");

@@ -62,7 +62,9 @@ struct Cell {
     uint32_t status;
 };
 
-SDF_HD double dabs(double x) { return x < 0.0 ? -x : x; }
+// (the builtin is a free source modifier of the fp64 instructions; a compare and
+// select took four instructions, 15% of a clip's)
+SDF_HD double dabs(double x) { return __builtin_fabs(x); }
 
 // 3x3 determinant of rows a, b, c and its permanent (|terms| summed)
 SDF_HD double det3(const double *a, const double *b, const double *c, double &perm) {
