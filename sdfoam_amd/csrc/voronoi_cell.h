@@ -62,8 +62,8 @@ struct Cell {
     uint32_t status;
 };
 
-// (the builtin is a free source modifier of the fp64 instructions; a compare and
-// select took four instructions, 15% of a clip's)
+// (the builtin is a source modifier of the fp64 instructions; a compare and
+// select took four instructions of its own)
 SDF_HD double dabs(double x) { return __builtin_fabs(x); }
 
 // 3x3 determinant of rows a, b, c and its permanent (|terms| summed)
