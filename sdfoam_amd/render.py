@@ -19,6 +19,9 @@ import torch
 
 from .pipeline import Pipeline
 
+# as defined: a function set on the class later is someone else's
+_OWN_BACKWARD = Pipeline.trace_backward
+
 
 class ErrorBox:
     """Carrier for per-ray error in and per-point error out
@@ -88,8 +91,8 @@ class TraceRays(torch.autograd.Function):
         options = dict(alpha_mode="sdfoam" if ctx.use_sdfoam else "standard", inv_s=ctx.inv_s,
                        sdf_channel=ctx.sdf_channel)
         # this package's pipeline zeroes the non-finite gradients as it writes
-        # them; another's, or an overridden trace_backward, is called as is
-        own = getattr(ctx.pipeline.trace_backward, "__func__", None) is Pipeline.trace_backward
+        # them; another's, or a replaced trace_backward, is called as is
+        own = getattr(ctx.pipeline.trace_backward, "__func__", None) is _OWN_BACKWARD
         if own:
             results = ctx.pipeline._backward(*args, **options, autograd=True)
         else:
