@@ -280,7 +280,10 @@ typedef struct sdf_trace_plan {
     void *grad_accum;          /* device memory, 256-byte aligned, or NULL */
     size_t grad_accum_bytes;   /* >= sdf_grad_accum_bytes(sh_degree, num_points); with
                                   8 * num_points (rounded up to 16) more, point errors
-                                  are summed there in fp64 */
+                                  are summed there in fp64; with sdf_grad_sums_bytes(
+                                  sh_degree, num_points) more, so are the sharpness'
+                                  gradient and the gradients of cells that rays start in,
+                                  and several lanes share a ray where rays are few */
     uint32_t scratch_ready;    /* backward: nonzero if `scratch` already holds this
                                   scene's offset table (the forward over the same
                                   scene filled it); the backward then skips
@@ -318,6 +321,9 @@ size_t sdf_cell_table_bytes(int sh_degree, int attr_type, uint32_t num_points);
 
 /* Bytes of the backward's gradient accumulator (0 for an invalid degree). */
 size_t sdf_grad_accum_bytes(int sh_degree, uint32_t num_points);
+
+/* Bytes of the fp64 sums behind the accumulator's rows (0: bad degree). */
+size_t sdf_grad_sums_bytes(int sh_degree, uint32_t num_points);
 
 /* Scratch bytes of sdf_ray_order. */
 size_t sdf_ray_order_scratch_bytes(uint32_t num_points, uint32_t num_rays);

@@ -36,6 +36,7 @@ EXPORTS = (
     "sdf_walk_record_pool_bytes",
     "sdf_walk_record_full_chunks",
     "sdf_grad_accum_bytes",
+    "sdf_grad_sums_bytes",
     "sdf_cell_table_bytes",
     "sdf_start_points_scratch_bytes",
     "sdf_start_points",
@@ -198,6 +199,8 @@ def lib() -> C.CDLL:
     L.sdf_walk_record_full_chunks.argtypes = [U32, U32, U32]
     L.sdf_grad_accum_bytes.restype = SZ
     L.sdf_grad_accum_bytes.argtypes = [C.c_int, U32]
+    L.sdf_grad_sums_bytes.restype = SZ
+    L.sdf_grad_sums_bytes.argtypes = [C.c_int, U32]
     L.sdf_start_points_scratch_bytes.restype = SZ
     L.sdf_start_points_scratch_bytes.argtypes = [U32]
     L.sdf_start_points.argtypes = [P, U32, P, U32, P, P, P, SZ, P]

@@ -275,6 +275,7 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (rc != SDF_OK) return rc;
     float *accum = nullptr;
     double *error_sums = nullptr;
+    StartSums *start_sums = nullptr;
     if (plan && plan->grad_accum) {
         const size_t need = sdf_grad_accum_bytes(sh_degree, num_points);
         if (plan->grad_accum_bytes < need)
@@ -286,6 +287,9 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
         if (ray_error && point_error &&
             plan->grad_accum_bytes >= need + error_sums_bytes(num_points))
             error_sums = reinterpret_cast<double *>(static_cast<char *>(plan->grad_accum) + need);
+        if (num_rays > 0 && plan->grad_accum_bytes >= need + sdf_grad_sums_bytes(sh_degree, num_points))
+            start_sums = reinterpret_cast<StartSums *>(static_cast<char *>(plan->grad_accum) + need +
+                                                       error_sums_bytes(num_points));
     }
     const uint32_t outputs = plan ? plan->outputs : 0u;
     if ((outputs & SDF_OUTPUTS_FRESH) != 0 && (!accum || num_rays == 0))
@@ -302,13 +306,6 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
         if (e != hipSuccess) return hip_fail(e, "prefetch_adjacent_diff");
     }
     if (num_rays == 0) return SDF_OK;
-    if (accum) {
-        tbegin(SDF_KERNEL_GRAD_CLEAR, s);
-        e = launch_grad_clear(sh_degree, accum, num_points, error_sums != nullptr,
-                              (outputs & SDF_OUTPUTS_FRESH) ? sharpness_grad : nullptr, s);
-        tend(s);
-        if (e != hipSuccess) return hip_fail(e, "gradient accumulator clear");
-    }
     BwdArgs a = {};
     a.record = rec;
     a.order = order;
@@ -333,6 +330,13 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     a.sharpness_grad = sharpness_grad;
     a.accum = accum;
     a.error_sums = error_sums;
+    a.start_sums = start_sums;
+    if (accum) {
+        tbegin(SDF_KERNEL_GRAD_CLEAR, s);
+        e = launch_grad_clear(sh_degree, a, (outputs & SDF_OUTPUTS_FRESH) && sharpness_grad, s);
+        tend(s);
+        if (e != hipSuccess) return hip_fail(e, "gradient accumulator clear");
+    }
     tbegin(SDF_KERNEL_BACKWARD, s);
     e = launch_backward(sh_degree, a, neus, false, half, s);
     tend(s);
@@ -340,7 +344,8 @@ int trace_backward_impl(const sdf_trace_plan *plan, int sh_degree,
     if (accum) {
         tbegin(SDF_KERNEL_GRAD_FINALIZE, s);
         e = launch_grad_finalize(sh_degree, accum, num_points, attribute_grad, points_grad,
-                                 a.point_error, sharpness_grad, error_sums, outputs, half, s);
+                                 a.point_error, sharpness_grad, error_sums, start_sums, outputs,
+                                 half, s);
         tend(s);
         if (e != hipSuccess) return hip_fail(e, "gradient accumulator finalize");
     }
@@ -408,6 +413,11 @@ size_t sdf_cell_table_bytes(int sh_degree, int attr_type, uint32_t num_points) {
 size_t sdf_grad_accum_bytes(int sh_degree, uint32_t num_points) {
     if (sh_degree < 0 || sh_degree > 3) return 0;
     return (size_t)num_points * accum_stride(sh_degree) * sizeof(float);
+}
+
+size_t sdf_grad_sums_bytes(int sh_degree, uint32_t num_points) {
+    if (sh_degree < 0 || sh_degree > 3) return 0;
+    return error_sums_bytes(num_points) + start_sums_bytes(sh_degree);
 }
 
 size_t sdf_trace_scratch_bytes(uint32_t num_points, uint32_t adjacency_size) {

@@ -158,6 +158,25 @@ struct FwdArgs {
     uint32_t cells_stride;
 };
 
+// Sums that many rays add to, in fp64: the sharpness' gradient, and the rows of
+// up to kStartRows cells that sampled rays start in or cross first.  Rays that
+// share a camera share those cells: each gets a term from every wavefront, so
+// its fp32 sum would lose more the fewer rays a wavefront holds.  Against 64-bit
+// sums of the same terms, over 160 traces (4k to 400k points, 6k to 1.7M rays,
+// geometric means, one lane per ray with fp32 sums = 1): more lanes with fp32
+// sums 1.18 (attributes), 1.12 (positions) and 2.0 (sharpness), with these 1.00,
+// 0.94 and below 0.01.  They cost the backward 0.28 of 19.0 ms (1M random rays, 2M
+// points) and, for 64x64 rays, 6 of 91 us.  Every row is there kStartCopies
+// times (blocks take turns): one copy alone took 3% of a 1600x1200 backward
+// waiting for atomics.  Zeroed but for `cells`.
+constexpr uint32_t kStartRows = 64, kStartCopies = 8;
+
+struct StartSums {
+    uint32_t cells[kStartRows]; // all different; kNoIndex: none
+    double sharpness, pad;
+    double rows[]; // [kStartRows][kStartCopies][accum_stride(L)], as the accumulator's
+};
+
 struct BwdArgs {
     WalkRecordArgs record;
     const uint32_t *order;
@@ -186,6 +205,9 @@ struct BwdArgs {
     // behind the rows: the point errors' fp64 sums [N] (error_sums_bytes), or
     // nullptr (the rows hold them)
     double *error_sums;
+    // behind those: the fp64 sums that all rays add to, or nullptr (the rows
+    // and sharpness_grad hold them)
+    StartSums *start_sums;
     // walk statistics (STATS instantiation only)
     uint64_t *visit_hash;
     uint32_t *steps;
@@ -254,21 +276,27 @@ __host__ inline uint64_t error_sums_bytes(uint32_t num_points) {
     return (8ull * num_points + 15) / 16 * 16;
 }
 
-// Clears num_points rows of the accumulator, the point errors' sums behind
-// them (error_sums), and sharpness_grad[0] if given.
-hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, bool error_sums,
-                             float *sharpness_grad, hipStream_t stream);
+// Bytes of a StartSums.
+__host__ inline uint64_t start_sums_bytes(int L) {
+    return sizeof(StartSums) + 8ull * kStartRows * kStartCopies * accum_stride(L);
+}
+
+// Clears what launch_backward(L, a) adds to beside the outputs: the
+// accumulator's rows, error_sums and start_sums (and chooses its cells; none
+// where a wavefront holds 64 rays); with clear_sharpness sharpness_grad[0] too.
+hipError_t launch_grad_clear(int L, const BwdArgs &a, bool clear_sharpness, hipStream_t stream);
 
 // attribute_grad [N, D] += rows[:, :D]; points_grad [N, 3] += rows[:, D:D+3];
 // point_error [N] += rows[:, D+3], or error_sums where given (point_error may
-// be nullptr).  attr_grad and
+// be nullptr).  start_sums, where given, holds the rest of its cells' rows and
+// sharpness_grad[0].  attr_grad and
 // point_error are fp16 when `half` (the sum is rounded once), else fp32.
 // outputs: SDF_OUTPUTS_* bits; with SDF_OUTPUTS_FINITE sharpness_grad[0] too
 // becomes 0 where it is not finite.
 hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, void *attr_grad,
                                 float *points_grad, void *point_error, float *sharpness_grad,
-                                const double *error_sums, uint32_t outputs, bool half,
-                                hipStream_t stream);
+                                const double *error_sums, const StartSums *start_sums,
+                                uint32_t outputs, bool half, hipStream_t stream);
 
 hipError_t launch_backward(int L, const BwdArgs &a, bool neus, bool stats, bool half,
                            hipStream_t stream);

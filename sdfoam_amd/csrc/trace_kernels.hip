@@ -903,17 +903,22 @@ __device__ __forceinline__ void publish_step(WaveTables<L, PE> &tb, StepEntries 
 // the rows).  They are sums of one sign, and a cell that all rays cross gets one
 // term per wavefront: with fewer rays per wavefront there are more of them to
 // round, 1.2e-6 against 0.7e-6 of the sums at 400x400 rays in fp32.
+// start_rows (ACC): the rows of the cells start_cells (in LDS) go there instead
+// (this block's copy of row 0), or NULL.
 // ALSO_LAST: the last channel is an SH component too (sdf_channel < 3 nsh).
-template <int L, bool PE, typename AT, bool ACC, bool ALSO_LAST>
+template <int L, bool PE, typename AT, bool ACC, bool ALSO_LAST, int G>
 __device__ __forceinline__ void grouped_pass_impl(StepEntries &e, const OwnerLane &ow,
                                                   WaveTables<L, PE> &tb, void *__restrict__ attr_grad,
                                                   void *__restrict__ point_error,
                                                   float *__restrict__ points_grad,
                                                   float *__restrict__ row,
-                                                  double *__restrict__ error_sums) {
+                                                  double *__restrict__ error_sums,
+                                                  double *__restrict__ start_rows,
+                                                  const uint32_t *start_cells) {
     constexpr int D = 1 + 3 * (L + 1) * (L + 1);
     const uint32_t lane = lane_id();
     const float *last = tb.rec() + 3 * kPitch;
+    const uint32_t start_cell = ACC && G > 1 ? start_cells[lane] : kNoIndex;
     uint64_t todo[kWindow], flushing[kWindow];
 #pragma unroll
     for (int s = 0; s < kWindow; ++s) {
@@ -949,7 +954,15 @@ __device__ __forceinline__ void grouped_pass_impl(StepEntries &e, const OwnerLan
             acc = acc + sum_members<ALSO_LAST>(grp[s], tb.buf, ow, s, ls);
         }
         if constexpr (ACC) {
-            if (ow.row_active) atomicAdd(row + (uint64_t)c * accum_stride(L), acc);
+            const uint64_t at = G > 1 ? __ballot(start_cell == c) : 0ull;
+            if (at) { // uniform
+                if (ow.row_active)
+                    atomicAdd(start_rows + (uint32_t)first_lane(at) * (kStartCopies * accum_stride(L)) +
+                                  ow.row_off,
+                              (double)acc);
+            } else if (ow.row_active) {
+                atomicAdd(row + (uint64_t)c * accum_stride(L), acc);
+            }
             if constexpr (PE) {
                 if (error_sums && lane == 63u) atomicAdd(error_sums + c, (double)acc);
             }
@@ -985,39 +998,57 @@ struct PassTarget {
     float *points_grad;
     float *row;         // accumulator: this lane's element of cell 0's row, or nullptr
     double *error_sums; // beside the rows: the point errors' sums, or nullptr
+    double *start_rows;          // beside the rows: this block's copy of StartSums' first row
+    const uint32_t *start_cells; // their cells, in LDS
     bool also_last;     // some owner lane adds the last channel to an SH component
 };
 
-template <int L, bool PE, typename AT>
+template <int L, bool PE, typename AT, int G>
 __device__ __forceinline__ void grouped_pass(StepEntries &e, const OwnerLane &ow,
                                              WaveTables<L, PE> &tb, const PassTarget &t) {
     __builtin_amdgcn_wave_barrier();
     if (t.row) {
         if (t.also_last)
-            grouped_pass_impl<L, PE, AT, true, true>(e, ow, tb, t.attr_grad, t.point_error,
-                                                     t.points_grad, t.row, t.error_sums);
+            grouped_pass_impl<L, PE, AT, true, true, G>(e, ow, tb, t.attr_grad, t.point_error,
+                                                        t.points_grad, t.row, t.error_sums,
+                                                        t.start_rows, t.start_cells);
         else
-            grouped_pass_impl<L, PE, AT, true, false>(e, ow, tb, t.attr_grad, t.point_error,
-                                                      t.points_grad, t.row, t.error_sums);
+            grouped_pass_impl<L, PE, AT, true, false, G>(e, ow, tb, t.attr_grad, t.point_error,
+                                                         t.points_grad, t.row, t.error_sums,
+                                                         t.start_rows, t.start_cells);
     } else {
         if (t.also_last)
-            grouped_pass_impl<L, PE, AT, false, true>(e, ow, tb, t.attr_grad, t.point_error,
-                                                      t.points_grad, t.row, t.error_sums);
+            grouped_pass_impl<L, PE, AT, false, true, G>(e, ow, tb, t.attr_grad, t.point_error,
+                                                         t.points_grad, nullptr, nullptr, nullptr,
+                                                         nullptr);
         else
-            grouped_pass_impl<L, PE, AT, false, false>(e, ow, tb, t.attr_grad, t.point_error,
-                                                       t.points_grad, t.row, t.error_sums);
+            grouped_pass_impl<L, PE, AT, false, false, G>(e, ow, tb, t.attr_grad, t.point_error,
+                                                          t.points_grad, nullptr, nullptr, nullptr,
+                                                          nullptr);
     }
     __builtin_amdgcn_wave_barrier();
 }
 
-template <int L>
-__device__ __forceinline__ PassTarget pass_target(const BwdArgs &a, const OwnerLane &ow) {
+// start_cells: kStartRows words of LDS (G > 1), one copy for the block: every
+// wavefront writes the same values before it reads them.
+template <int L, int G>
+__device__ __forceinline__ PassTarget pass_target(const BwdArgs &a, const OwnerLane &ow,
+                                                  uint32_t *start_cells) {
+    static_assert(kStartRows == 64, "one start cell per lane");
+    if constexpr (G > 1) {
+        start_cells[lane_id()] = a.start_sums ? a.start_sums->cells[lane_id()] : kNoIndex;
+        __builtin_amdgcn_wave_barrier();
+    }
     PassTarget t;
     t.attr_grad = a.attr_grad;
     t.point_error = a.point_error;
     t.points_grad = a.points_grad;
     t.row = a.accum ? a.accum + ow.row_off : nullptr;
     t.error_sums = a.error_sums;
+    t.start_rows = G > 1 && a.start_sums
+                       ? a.start_sums->rows + blockIdx.x % kStartCopies * accum_stride(L)
+                       : nullptr;
+    t.start_cells = start_cells;
     t.also_last = __ballot(ow.also_last) != 0ull;
     return t;
 }
@@ -1077,6 +1108,7 @@ backward_sdf_kernel(BwdArgs a) {
     constexpr int nsh = (L + 1) * (L + 1);
     constexpr int D = 1 + 3 * nsh;
     __shared__ WaveTables<L, PE> tables[kBlock / 64];
+    __shared__ uint32_t start_cells[kStartRows];
     const BackwardLane bl = backward_lane<G>(a);
     const bool valid = bl.valid;
     const uint32_t ray_idx = bl.ray;
@@ -1096,7 +1128,7 @@ backward_sdf_kernel(BwdArgs a) {
     const int32_t sdf_ch = a.settings.sdf_channel >= 0 ? a.settings.sdf_channel : D - 1;
     const bool write_sdf = a.settings.sdf_channel >= 0;
     const OwnerLane owner = owner_lane<L, PE>(write_sdf ? sdf_ch : -1, a.error_sums != nullptr);
-    const PassTarget target = pass_target<L>(a, owner);
+    const PassTarget target = pass_target<L, G>(a, owner, start_cells);
     const float thr = a.settings.weight_threshold;
     const uint32_t Q = a.num_quantiles;
     const float *rq = (valid && a.quantiles) ? a.quantiles + (uint64_t)ray_idx * Q : nullptr;
@@ -1265,7 +1297,7 @@ backward_sdf_kernel(BwdArgs a) {
             // steps go out every kWindow trips
             if (ents.pend && (si.stepped || !ws.alive))
                 complete_entry<L, PE>(ents, si.stepped && flush, flush_g, tb);
-            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
+            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT, G>(ents, owner, tb, target);
             if (si.stepped && (G == 1 || turn++ % G == bl.sub))
                 publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dsdf, pe);
         }
@@ -1275,7 +1307,7 @@ backward_sdf_kernel(BwdArgs a) {
         // steps not applied when the walks ended
         const float zero3[3] = {0.0f, 0.0f, 0.0f};
         if (ents.pend) complete_entry<L, PE>(ents, false, zero3, tb);
-        grouped_pass<L, PE, AT>(ents, owner, tb, target);
+        grouped_pass<L, PE, AT, G>(ents, owner, tb, target);
     }
 
     if constexpr (STATS) {
@@ -1288,7 +1320,12 @@ backward_sdf_kernel(BwdArgs a) {
     } else {
         if (a.sharpness_grad) {
             const float v = wave_sum(G == 1 || bl.sub == 0 ? sharp_acc : 0.0f);
-            if (lane == 0 && v != 0.0f) atomicAdd(a.sharpness_grad, v);
+            if (lane == 0 && v != 0.0f) {
+                if (a.start_sums)
+                    atomicAdd(&a.start_sums->sharpness, (double)v);
+                else
+                    atomicAdd(a.sharpness_grad, v);
+            }
         }
     }
 }
@@ -1301,6 +1338,7 @@ backward_density_kernel(BwdArgs a) {
     constexpr int nsh = (L + 1) * (L + 1);
     constexpr int D = 1 + 3 * nsh;
     __shared__ WaveTables<L, PE> tables[kBlock / 64];
+    __shared__ uint32_t start_cells[kStartRows];
     const BackwardLane bl = backward_lane<G>(a);
     const bool valid = bl.valid;
     const uint32_t ray_idx = bl.ray;
@@ -1317,7 +1355,7 @@ backward_density_kernel(BwdArgs a) {
     const float *sh = tb.y() + lane; // this ray's SH basis, in LDS (stride kPitch)
 
     const OwnerLane owner = owner_lane<L, PE>(D - 1, a.error_sums != nullptr);
-    const PassTarget target = pass_target<L>(a, owner);
+    const PassTarget target = pass_target<L, G>(a, owner, start_cells);
     const float thr = a.settings.weight_threshold;
     const uint32_t Q = a.num_quantiles;
     const float *rq = (valid && a.quantiles) ? a.quantiles + (uint64_t)ray_idx * Q : nullptr;
@@ -1496,7 +1534,7 @@ backward_density_kernel(BwdArgs a) {
         if constexpr (!STATS) {
             if (ents.pend && (si.stepped || !ws.alive))
                 complete_entry<L, PE>(ents, si.stepped && flush, flush_g, tb);
-            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT>(ents, owner, tb, target);
+            if (trip % (kWindow * G) == 0) grouped_pass<L, PE, AT, G>(ents, owner, tb, target);
             if (si.stepped && (G == 1 || turn++ % G == bl.sub))
                 publish_step<L, PE>(tb, ents, ws.cell, dr, dg, db, dds, pe);
         }
@@ -1524,7 +1562,7 @@ backward_density_kernel(BwdArgs a) {
     if constexpr (!STATS) {
         const float zero3[3] = {0.0f, 0.0f, 0.0f};
         if (ents.pend) complete_entry<L, PE>(ents, false, zero3, tb);
-        grouped_pass<L, PE, AT>(ents, owner, tb, target);
+        grouped_pass<L, PE, AT, G>(ents, owner, tb, target);
     }
 
     if constexpr (STATS) {
@@ -1576,7 +1614,11 @@ int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered) {
     return num_rays <= 163840u ? 2 : 1;
 }
 
-static int backward_lanes(uint32_t num_rays, uint32_t num_points) {
+static int backward_lanes(const BwdArgs &a) {
+    const uint32_t num_rays = a.num_rays, num_points = a.scene.num_points;
+    // without the fp64 sums a cell that all rays cross would take more
+    // rounded terms from more lanes per ray
+    if (!a.start_sums || (a.point_error && !a.error_sums)) return 1;
     if (num_rays < 2ull * num_points) {
         if (num_rays <= 16384u) return 16;
         if (num_rays <= 49152u) return 8;
@@ -1838,9 +1880,7 @@ static hipError_t launch_backward_G(const BwdArgs &a, bool neus, hipStream_t str
 template <int L, typename AT>
 static hipError_t launch_backward_L(const BwdArgs &a, bool neus, bool stats, hipStream_t stream) {
     if (!stats) {
-        // (fp16 gradients without the accumulator keep their roundings)
-        const bool keep = sizeof(AT) == 2 && !a.accum;
-        switch (keep ? 1 : backward_lanes(a.num_rays, a.scene.num_points)) {
+        switch (backward_lanes(a)) {
         case 16: return launch_backward_G<L, AT, 16>(a, neus, stream);
         case 8: return launch_backward_G<L, AT, 8>(a, neus, stream);
         case 4: return launch_backward_G<L, AT, 4>(a, neus, stream);
@@ -1880,13 +1920,52 @@ hipError_t launch_backward(int L, const BwdArgs &a, bool neus, bool stats, bool 
 
 constexpr uint32_t kAccumBlocks = 16384; // grid-stride cap of the two passes
 
-__global__ __launch_bounds__(kBlock) void grad_clear_kernel(float4 *__restrict__ rows,
-                                                            uint64_t n4,
-                                                            float *__restrict__ sharpness_grad) {
-    if (sharpness_grad && blockIdx.x == 0 && threadIdx.x == 0) sharpness_grad[0] = 0.0f;
+// The cells of StartSums, one per lane of a wavefront: the first 4 cells of 16
+// rays of an image (one camera: its rays share their first cells), the first 2
+// of 32 rays of a batch (several cameras).  The cells after the first are in
+// the walk record.
+__device__ __forceinline__ uint32_t start_cell_of(const BwdArgs &a) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool image = a.settings.ray_image_width != 0 && !a.order;
+    const uint32_t deep = image ? 4u : 2u;
+    const uint32_t sample = lane / deep, j = lane % deep;
+    const uint32_t rows = image ? 4u * a.num_tiles : (a.num_rays + 63u) / 64u; // of 64 rays
+    const uint32_t row = (uint32_t)((2ull * sample + 1ull) * rows / (2ull * (kStartRows / deep)));
+    bool valid;
+    const uint32_t ray = ray_at(row, 0, a.num_rays, a.settings.ray_image_width, a.num_tiles, valid,
+                                a.order);
+    uint32_t c = valid ? a.start[ray] : kNoIndex;
+    if (valid && j > 0) {
+        c = kNoIndex;
+        if (a.record.entries && j - 1u < a.record.budget) {
+            const uint64_t i = record_slot(
+                a.record, a.record.chunks + (uint64_t)row * chunk_slots(a.record.budget), j - 1u, 0);
+            if (i != ~0ull) c = a.record.entries[i].x; // after the walk's end: anything
+            if (c < kNoIndex - 1u) c &= ~kWalkDiffers;
+        }
+    }
+    if (c >= a.scene.num_points) c = kNoIndex;
+    // keep the first of equal ones
+    bool dup = false;
+    for (uint32_t k = 0; k < kStartRows; ++k) dup = dup || (k < lane && readlane_u(c, (int)k) == c);
+    return dup ? kNoIndex : c;
+}
+
+__global__ __launch_bounds__(kBlock) void grad_clear_kernel(BwdArgs a, uint64_t n4, uint32_t stride,
+                                                            bool start_rows, bool clear_sharpness) {
+    if (clear_sharpness && blockIdx.x == 0 && threadIdx.x == 0) a.sharpness_grad[0] = 0.0f;
+    if (a.start_sums && blockIdx.x == 0 && threadIdx.x < 64u) {
+        a.start_sums->cells[threadIdx.x] = start_rows ? start_cell_of(a) : kNoIndex;
+        if (threadIdx.x == 0) a.start_sums->sharpness = 0.0;
+    }
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n4; i += step)
-        rows[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    float4 *rows = reinterpret_cast<float4 *>(a.accum);
+    for (uint64_t i = i0; i < n4; i += step) rows[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (a.start_sums && start_rows) {
+        for (uint64_t i = i0; i < kStartRows * kStartCopies * stride; i += step)
+            a.start_sums->rows[i] = 0.0;
+    }
 }
 
 // One thread per 16 bytes of a row (the row's padding past D + 4 floats
@@ -1903,7 +1982,8 @@ template <int L, typename AT, bool FRESH>
 __global__ __launch_bounds__(kBlock) void grad_finalize_kernel(
     const float4 *__restrict__ rows, uint32_t num_points, AT *__restrict__ attr_grad,
     float *__restrict__ points_grad, AT *__restrict__ point_error,
-    float *__restrict__ sharpness_grad, const double *__restrict__ error_sums, bool finite) {
+    float *__restrict__ sharpness_grad, const double *__restrict__ error_sums,
+    const StartSums *__restrict__ start_sums, bool finite) {
     constexpr uint32_t S4 = accum_stride(L) / 4;
     constexpr uint32_t D = 1 + 3 * (L + 1) * (L + 1);
     constexpr uint32_t Q = (D + 4 + 3) / 4; // quads of a row that hold data
@@ -1911,15 +1991,40 @@ __global__ __launch_bounds__(kBlock) void grad_finalize_kernel(
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     // NaN and infinities fail |x| <= FLT_MAX
     auto kept = [finite](float x) { return !finite || fabsf(x) <= 3.402823466e+38f; };
-    if (FRESH && sharpness_grad && blockIdx.x == 0 && threadIdx.x == 0 &&
-        !kept(sharpness_grad[0]))
-        sharpness_grad[0] = 0.0f;
-    for (uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x; t < total; t += step) {
+    if (sharpness_grad && blockIdx.x == 0 && threadIdx.x == 0) {
+        float x = FRESH && start_sums ? 0.0f : sharpness_grad[0];
+        if (start_sums) x += (float)start_sums->sharpness;
+        sharpness_grad[0] = !FRESH || kept(x) ? x : 0.0f;
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t start_cell = start_sums ? start_sums->cells[lane] : kNoIndex;
+    const bool any_start = __ballot(start_cell != kNoIndex) != 0ull;
+    // t0: the wavefront's first quad (every lane goes round the loop together)
+    for (uint64_t t0 = (uint64_t)blockIdx.x * kBlock + (threadIdx.x - lane); t0 < total;
+         t0 += step) {
+        const uint64_t t = t0 + lane;
+        // the start cells among the wavefront's
+        uint64_t hot = !any_start ? 0ull
+                                  : __ballot(start_cell >= t0 / S4 &&
+                                             start_cell <= (t0 + 63u) / S4 &&
+                                             start_cell != kNoIndex);
         const uint32_t q = (uint32_t)(t % S4);
-        if (q >= Q) continue;
-        const float4 v4 = rows[t];
-        float v[4] = {v4.x, v4.y, v4.z, v4.w};
         const uint64_t c = t / S4;
+        double add[4] = {0.0, 0.0, 0.0, 0.0};
+        for (; hot; hot &= hot - 1ull) {
+            const uint32_t k = (uint32_t)__builtin_ctzll(hot);
+            if (readlane_u(start_cell, (int)k) == c) {
+                for (uint32_t s = 0; s < kStartCopies; ++s) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j)
+                        add[j] += start_sums->rows[((k * kStartCopies + s) * S4 + q) * 4u + j];
+                }
+            }
+        }
+        if (t >= total || q >= Q) continue;
+        const float4 v4 = rows[t];
+        float v[4] = {(float)((double)v4.x + add[0]), (float)((double)v4.y + add[1]),
+                      (float)((double)v4.z + add[2]), (float)((double)v4.w + add[3])};
         if (error_sums && q == (D + 3) / 4) v[(D + 3) % 4] = (float)error_sums[c];
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
@@ -1954,13 +2059,13 @@ static inline dim3 accum_grid(uint64_t threads) {
     return dim3((unsigned)(b < kAccumBlocks ? (b ? b : 1) : kAccumBlocks));
 }
 
-hipError_t launch_grad_clear(int L, float *accum, uint32_t num_points, bool error_sums,
-                             float *sharpness_grad, hipStream_t stream) {
+hipError_t launch_grad_clear(int L, const BwdArgs &a, bool clear_sharpness, hipStream_t stream) {
     if (L < 0 || L > 3) return hipErrorInvalidValue;
-    const uint64_t n4 = (uint64_t)num_points * accum_stride(L) / 4 +
-                        (error_sums ? error_sums_bytes(num_points) / 16 : 0);
-    hipLaunchKernelGGL(grad_clear_kernel, accum_grid(n4), dim3(kBlock), 0, stream,
-                       reinterpret_cast<float4 *>(accum), n4, sharpness_grad);
+    const uint32_t n = a.scene.num_points;
+    const uint64_t n4 = (uint64_t)n * accum_stride(L) / 4 +
+                        (a.error_sums ? error_sums_bytes(n) / 16 : 0);
+    hipLaunchKernelGGL(grad_clear_kernel, accum_grid(n4), dim3(kBlock), 0, stream, a, n4,
+                       accum_stride(L), backward_lanes(a) > 1, clear_sharpness);
     return hipGetLastError();
 }
 
@@ -1968,7 +2073,8 @@ template <int L, typename AT>
 static hipError_t launch_grad_finalize_L(const float *accum, uint32_t num_points, void *attr_grad,
                                          float *points_grad, void *point_error,
                                          float *sharpness_grad, const double *error_sums,
-                                         uint32_t outputs, hipStream_t stream) {
+                                         const StartSums *start_sums, uint32_t outputs,
+                                         hipStream_t stream) {
     const dim3 grid = accum_grid((uint64_t)num_points * accum_stride(L) / 4);
     const float4 *rows = reinterpret_cast<const float4 *>(accum);
     AT *ag = static_cast<AT *>(attr_grad);
@@ -1976,28 +2082,30 @@ static hipError_t launch_grad_finalize_L(const float *accum, uint32_t num_points
     const bool finite = (outputs & SDF_OUTPUTS_FINITE) != 0;
     if (outputs & SDF_OUTPUTS_FRESH) {
         hipLaunchKernelGGL((grad_finalize_kernel<L, AT, true>), grid, dim3(kBlock), 0, stream, rows,
-                           num_points, ag, points_grad, pe, sharpness_grad, error_sums, finite);
+                           num_points, ag, points_grad, pe, sharpness_grad, error_sums,
+                           start_sums, finite);
     } else {
         hipLaunchKernelGGL((grad_finalize_kernel<L, AT, false>), grid, dim3(kBlock), 0, stream, rows,
-                           num_points, ag, points_grad, pe, nullptr, error_sums, false);
+                           num_points, ag, points_grad, pe, start_sums ? sharpness_grad : nullptr,
+                           error_sums, start_sums, false);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_grad_finalize(int L, const float *accum, uint32_t num_points, void *attr_grad,
                                 float *points_grad, void *point_error, float *sharpness_grad,
-                                const double *error_sums, uint32_t outputs, bool half,
-                                hipStream_t stream) {
+                                const double *error_sums, const StartSums *start_sums,
+                                uint32_t outputs, bool half, hipStream_t stream) {
 #define SDF_FINALIZE(N)                                                                        \
     case N:                                                                                    \
         return half ? launch_grad_finalize_L<N, _Float16>(accum, num_points, attr_grad,        \
                                                           points_grad, point_error,            \
-                                                          sharpness_grad, error_sums, outputs, \
-                                                          stream)                              \
+                                                          sharpness_grad, error_sums,          \
+                                                          start_sums, outputs, stream)         \
                     : launch_grad_finalize_L<N, float>(accum, num_points, attr_grad,           \
                                                        points_grad, point_error,               \
-                                                       sharpness_grad, error_sums, outputs,    \
-                                                       stream)
+                                                       sharpness_grad, error_sums, start_sums, \
+                                                       outputs, stream)
     switch (L) {
         SDF_FINALIZE(0);
         SDF_FINALIZE(1);

@@ -698,9 +698,9 @@ class Pipeline:
         desc.scratch_ready = 1 if table_ready else 0
         accum = None
         if grad_accum and num_rays > 0:
-            accum_bytes = int(_lib.lib().sdf_grad_accum_bytes(self._sh_degree, num_points))
-            if return_error:
-                accum_bytes += -(-8 * num_points // 16) * 16  # its fp64 sums
+            # with the fp64 sums behind the rows
+            accum_bytes = int(_lib.lib().sdf_grad_accum_bytes(self._sh_degree, num_points)
+                              + _lib.lib().sdf_grad_sums_bytes(self._sh_degree, num_points))
             accum = torch.empty(accum_bytes + 256, dtype=torch.uint8, device=dev)
             desc.grad_accum = (accum.data_ptr() + 255) & ~255
             desc.grad_accum_bytes = accum_bytes
