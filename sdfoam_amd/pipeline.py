@@ -660,7 +660,9 @@ class Pipeline:
 
         num_attr = attributes_c.size(0)
         make = torch.empty if fresh else torch.zeros
-        attr_grad = self._attr_buffer((num_attr, self.attribute_dim()), dev, zero=not fresh)
+        # (attributes may have rows past the points: points [N, K, 3])
+        attr_grad = self._attr_buffer((num_attr, self.attribute_dim()), dev,
+                                      zero=not fresh or num_attr != num_points)
         points_grad = make((num_points, 3), dtype=rays_c.dtype, device=dev)
         # the kernels write the first element of the sharpness' gradient
         sharpness_grad = (make if sharpness.numel() == 1 else torch.zeros)(
