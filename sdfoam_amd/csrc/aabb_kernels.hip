@@ -225,7 +225,8 @@ __device__ void nn_load_top(const float *__restrict__ tree, uint32_t td, NNShare
 // Nearest point to q for the whole wavefront (the result is uniform), over
 // the tree of depth td (points padded to 2^td).  NaN lower bounds mark nodes
 // that are taken, outside the group or not comparable (NaN query): a node is
-// pending while lb <= best.  0 when no point has a distance (NaN query).
+// pending while lb < best, or lb == best and it holds a smaller index than the
+// best (its first one).  0 when no point has a distance (NaN query).
 __device__ uint32_t nn_wave(const float *__restrict__ points, const float *__restrict__ tree,
                             uint32_t num_points, uint32_t td, float qx, float qy, float qz,
                             NNShared &sh, uint32_t wave) {
@@ -271,7 +272,10 @@ __device__ uint32_t nn_wave(const float *__restrict__ points, const float *__res
     while (k >= 0) {
         __builtin_amdgcn_wave_barrier();
         const float lb = lbs[k][lane];
-        const bool pending = lb <= best;
+        const uint32_t d = 6u * (uint32_t)(k + 1);
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)first_of, k);
+        const bool pending =
+            lb < best || (lb == best && ((uint64_t)(first + lane) << (td - d)) < best_idx);
         float bl = pending ? lb : kInf;
         uint32_t bi = pending ? lane : 64u;
         wave_argmin(bl, bi);
@@ -280,8 +284,7 @@ __device__ uint32_t nn_wave(const float *__restrict__ points, const float *__res
             continue;
         }
         if (lane == bi) lbs[k][lane] = kNaN; // taken
-        const uint32_t d = 6u * (uint32_t)(k + 1);
-        const uint32_t node = (uint32_t)__builtin_amdgcn_readlane((int)first_of, k) + bi;
+        const uint32_t node = first + bi;
         const uint32_t dc = d + 6 < td ? d + 6 : td;
         const uint32_t cfirst = node << (dc - d);
         const uint32_t csize = 1u << (dc - d);
