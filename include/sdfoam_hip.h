@@ -419,9 +419,10 @@ int sdf_nn(const float *points, const float *aabb_tree, const float *queries,
            void *stream);
 
 /* sdf_nn with scratch, for the same results sooner: few points times queries
- * are scanned, else points and queries are sorted along a curve for the call
- * (a stream in capture searches the tree as sdf_nn does).  scratch:
- * sdf_nn_scratch_bytes(num_points, num_queries), 256-byte aligned. */
+ * are scanned, few points searched by the tree as sdf_nn does, else points and
+ * queries are sorted along a curve for the call (a stream in capture searches
+ * the tree).  scratch: sdf_nn_scratch_bytes(num_points, num_queries), 256-byte
+ * aligned; 0 bytes: none is needed. */
 size_t sdf_nn_scratch_bytes(uint32_t num_points, uint32_t num_queries);
 int sdf_nn_planned(const float *points, const float *aabb_tree,
                    const float *queries, uint32_t num_points,

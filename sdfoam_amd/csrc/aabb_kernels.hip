@@ -446,8 +446,8 @@ __global__ __launch_bounds__(kBlock) void start_unique_kernel(const uint32_t *__
 }
 
 // Nearest of the block's kBlock * kStartPts points (block `chunk` of them) to
-// each of the `count` positions q: per position one atomic of the smallest
-// (distance bits, index) into best.  Lanes keep their own smallest over their
+// each of the `count` positions q: per wavefront and position one atomic of the
+// smallest (distance bits, index) into slot (LDS).  Lanes keep their own smallest over their
 // points; the wave's smallest distance comes by DPP and its index from the
 // lanes that hold that distance (one, but for ties).
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
@@ -463,7 +463,7 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 
 __device__ __forceinline__ void brute_scan(const float *__restrict__ points, uint32_t num_points,
                                            uint32_t chunk, const float (*q)[3], uint32_t count,
-                                           unsigned long long *slot, uint64_t *__restrict__ best) {
+                                           unsigned long long *slot) {
     const uint64_t p0 = (uint64_t)chunk * kBlock * kStartPts + threadIdx.x;
     float px[kStartPts], py[kStartPts], pz[kStartPts];
 #pragma unroll
@@ -495,6 +495,10 @@ __device__ __forceinline__ void brute_scan(const float *__restrict__ points, uin
         if ((threadIdx.x & 63u) == 0)
             atomicMin(slot + u, (unsigned long long)least << 32 | first);
     }
+}
+
+__device__ __forceinline__ void brute_merge(uint32_t count, const unsigned long long *slot,
+                                            uint64_t *__restrict__ best) {
     __syncthreads();
     for (uint32_t u = threadIdx.x; u < count; u += kBlock)
         if (slot[u] != ~0ull) atomicMin(reinterpret_cast<unsigned long long *>(best) + u, slot[u]);
@@ -520,23 +524,26 @@ __global__ __launch_bounds__(kBlock) void start_brute_kernel(const float *__rest
         slot[u] = ~0ull;
     }
     __syncthreads();
-    brute_scan(points, num_points, blockIdx.x, q, count, slot, best);
+    brute_scan(points, num_points, blockIdx.x, q, count, slot);
+    brute_merge(count, slot, best);
 }
 
-// The same for nn's queries, kScanQueries of them per blockIdx.y (a block takes
-// its queries one after another, 0.7 us each: with 256 of them 1,000 queries
-// over 4,096 points took 192 us on 8 blocks).
+// The same for nn's queries, `per` of them (at most kScanQueries) per blockIdx.y.
+// A block takes its queries one after another, 0.7 us each, so few pairs go to
+// many blocks with few queries each: with 64 queries per block whatever the
+// sizes, 64 to 1,000 queries over 4,000 to 100k points took 53 us and more.
 constexpr uint32_t kScanQueries = 64;
+constexpr uint32_t kScanBlocks = 2048; // (8 per CU)
 
-__global__ __launch_bounds__(kBlock) void nn_brute_kernel(const float *__restrict__ points,
-                                                          uint32_t num_points,
-                                                          const float *__restrict__ queries,
-                                                          uint32_t num_queries,
-                                                          uint64_t *__restrict__ best) {
-    __shared__ float q[kScanQueries][3];
-    __shared__ unsigned long long slot[kScanQueries];
-    const uint32_t q0 = blockIdx.y * kScanQueries;
-    const uint32_t count = min(kScanQueries, num_queries - q0);
+// Up to this many points a block scans all of them and writes the results
+// itself: one launch instead of three.
+constexpr uint32_t kScanWhole = 4 * kBlock * kStartPts;
+
+__device__ __forceinline__ uint32_t scan_queries(const float *__restrict__ queries,
+                                                 uint32_t num_queries, uint32_t per, float (*q)[3],
+                                                 unsigned long long *slot) {
+    const uint32_t q0 = blockIdx.y * per;
+    const uint32_t count = min(per, num_queries - q0);
     if (threadIdx.x < count) {
         const uint32_t u = threadIdx.x;
 #pragma unroll
@@ -544,7 +551,36 @@ __global__ __launch_bounds__(kBlock) void nn_brute_kernel(const float *__restric
         slot[u] = ~0ull;
     }
     __syncthreads();
-    brute_scan(points, num_points, blockIdx.x, q, count, slot, best + q0);
+    return count;
+}
+
+__global__ __launch_bounds__(kBlock) void nn_whole_kernel(const float *__restrict__ points,
+                                                          uint32_t num_points,
+                                                          const float *__restrict__ queries,
+                                                          uint32_t num_queries, uint32_t per,
+                                                          uint32_t *__restrict__ indices) {
+    __shared__ float q[kScanQueries][3];
+    __shared__ unsigned long long slot[kScanQueries];
+    const uint32_t count = scan_queries(queries, num_queries, per, q, slot);
+    for (uint32_t chunk = 0; chunk * (kBlock * kStartPts) < num_points; ++chunk)
+        brute_scan(points, num_points, chunk, q, count, slot);
+    __syncthreads();
+    if (threadIdx.x < count) {
+        const unsigned long long s = slot[threadIdx.x];
+        indices[blockIdx.y * per + threadIdx.x] = s == ~0ull ? 0u : (uint32_t)s;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void nn_brute_kernel(const float *__restrict__ points,
+                                                          uint32_t num_points,
+                                                          const float *__restrict__ queries,
+                                                          uint32_t num_queries, uint32_t per,
+                                                          uint64_t *__restrict__ best) {
+    __shared__ float q[kScanQueries][3];
+    __shared__ unsigned long long slot[kScanQueries];
+    const uint32_t count = scan_queries(queries, num_queries, per, q, slot);
+    brute_scan(points, num_points, blockIdx.x, q, count, slot);
+    brute_merge(count, slot, best + blockIdx.y * per);
 }
 
 __global__ __launch_bounds__(kBlock) void nn_reset_kernel(uint64_t *__restrict__ best, uint32_t n) {
@@ -562,12 +598,25 @@ __global__ __launch_bounds__(kBlock) void nn_result_kernel(const uint64_t *__res
 hipError_t launch_nn_brute(const float *points, const float *queries, uint32_t num_points,
                            uint32_t num_queries, uint32_t *indices, uint64_t *best,
                            hipStream_t stream) {
+    const uint32_t chunks =
+        (uint32_t)(((uint64_t)num_points + kBlock * kStartPts - 1) / (kBlock * kStartPts));
+    const bool whole = num_points <= kScanWhole;
+    const uint32_t per = (uint32_t)std::min<uint64_t>(
+        kScanQueries,
+        std::max<uint64_t>(1, ((uint64_t)num_queries * (whole ? 1 : chunks) + kScanBlocks - 1) /
+                                  kScanBlocks));
+    // (nn_route scans for at most 65,536 queries, fewer the more points there are: at most
+    // 16,640 groups)
+    const dim3 grid(whole ? 1 : chunks, (num_queries + per - 1) / per);
+    if (whole) {
+        hipLaunchKernelGGL(nn_whole_kernel, grid, dim3(kBlock), 0, stream, points, num_points,
+                           queries, num_queries, per, indices);
+        return hipGetLastError();
+    }
     const dim3 per_query((num_queries + kBlock - 1) / kBlock);
-    const dim3 grid((uint32_t)(((uint64_t)num_points + kBlock * kStartPts - 1) / (kBlock * kStartPts)),
-                    (num_queries + kScanQueries - 1) / kScanQueries);
     hipLaunchKernelGGL(nn_reset_kernel, per_query, dim3(kBlock), 0, stream, best, num_queries);
     hipLaunchKernelGGL(nn_brute_kernel, grid, dim3(kBlock), 0, stream, points, num_points, queries,
-                       num_queries, best);
+                       num_queries, per, best);
     hipLaunchKernelGGL(nn_result_kernel, per_query, dim3(kBlock), 0, stream, best, num_queries,
                        indices);
     return hipGetLastError();

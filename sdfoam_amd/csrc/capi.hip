@@ -1021,9 +1021,10 @@ int sdf_nn_planned(const float *points, const float *aabb_tree, const float *que
     hipStream_t s = static_cast<hipStream_t>(stream);
     // a captured graph holds no memset nodes, which the sorts would record
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool scans = nn_scans(num_points, num_queries);
-    if (!scans && hipStreamIsCapturing(s, &capture) == hipSuccess &&
-        capture != hipStreamCaptureStatusNone)
+    const NNRoute route = nn_route(num_points, num_queries);
+    if (route == NNRoute::kTree ||
+        (route == NNRoute::kSorted && hipStreamIsCapturing(s, &capture) == hipSuccess &&
+         capture != hipStreamCaptureStatusNone))
         return sdf_nn(points, aabb_tree, queries, num_points, num_queries, indices, stream);
     const size_t need = sdf_nn_scratch_bytes(num_points, num_queries);
     if (need == 0) return fail(SDF_E_HIP, "nn: the sort's scratch could not be sized");
@@ -1033,10 +1034,11 @@ int sdf_nn_planned(const float *points, const float *aabb_tree, const float *que
         return fail(SDF_E_INVALID, "scratch must be 256-byte aligned");
     tbegin(SDF_KERNEL_NN, s);
     const hipError_t e =
-        scans ? launch_nn_brute(points, queries, num_points, num_queries, indices,
-                                static_cast<uint64_t *>(scratch), s)
-              : launch_nn_sorted(points, aabb_tree, queries, num_points, num_queries, indices,
-                                 scratch, s);
+        route == NNRoute::kScan
+            ? launch_nn_brute(points, queries, num_points, num_queries, indices,
+                              static_cast<uint64_t *>(scratch), s)
+            : launch_nn_sorted(points, aabb_tree, queries, num_points, num_queries, indices,
+                               scratch, s);
     tend(s);
     if (e != hipSuccess) return hip_fail(e, "nn");
     return SDF_OK;

@@ -186,7 +186,7 @@ __device__ __forceinline__ void test_group(const Search &s, Nearest &b, uint64_t
 template <int LEVEL>
 __device__ __forceinline__ void descend(const Search &s, Nearest &b, uint64_t first) {
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t lb = kNever, low = kNoIndex;
+    uint32_t lb = kNever;
     if (first + lane < s.width[LEVEL]) {
         const float4 lo = s.boxes[2 * (s.start[LEVEL] + first + lane)];
         const float4 hi = s.boxes[2 * (s.start[LEVEL] + first + lane) + 1];
@@ -195,16 +195,19 @@ __device__ __forceinline__ void descend(const Search &s, Nearest &b, uint64_t fi
         const float dz = fmaxf(fmaxf(lo.z - b.z, 0.0f), b.z - hi.z);
         const float d = sqrtf(sdf_dot3(dx, dy, dz, dx, dy, dz));
         lb = __builtin_bit_cast(uint32_t, d);
-        low = __builtin_bit_cast(uint32_t, lo.w);
     }
     while (true) {
         const uint32_t least = wave_min_bits(lb);
-        if (least == kNever || least > b.dist) return;
         uint64_t next = __builtin_amdgcn_ballot_w64(lb == least);
-        if (least == b.dist) {
-            const uint32_t lowest = wave_min_bits(lb == least ? low : kNoIndex);
+        if (least >= b.dist) { // (kNever is above every distance)
+            if (least > b.dist) return;
+            // the indices are read where there is a tie
+            uint32_t low = kNoIndex;
+            if (lb == least)
+                low = __builtin_bit_cast(uint32_t, s.boxes[2 * (s.start[LEVEL] + first + lane)].w);
+            const uint32_t lowest = wave_min_bits(low);
             if (lowest >= b.id) return;
-            next = __builtin_amdgcn_ballot_w64(lb == least && low == lowest);
+            next = __builtin_amdgcn_ballot_w64(low == lowest);
         }
         const int at = __builtin_ctzll(next);
         if (lane == (uint32_t)at) lb = kNever; // taken
@@ -301,21 +304,45 @@ hipError_t sort_positions(const float *x, uint32_t n, const float *root, char *b
 
 } // namespace
 
-// Which way nn takes when it has scratch.  Scanning every point costs about
-// 0.7-0.9 ps per point and query (2,048 points per block from registers); the
-// sorted search costs the sorts and boxes and then little per query.  The line
-// is where the two meet: at 1M points 390 queries take 277 us scanned and 391
-// take 270 us sorted, at 100k points 1,600 take 131 us scanned and 113 us sorted, at
-// 4,096 points 32,000 take 109 us scanned and 33,100 take 114 us sorted.
-bool nn_scans(uint32_t num_points, uint32_t num_queries) {
-    // (the scan's grid has at most 65,535 groups of 64 queries)
-    return num_queries < (1u << 22) &&
-           (uint64_t)num_points * num_queries <= (1ull << 27) + 256ull * num_points;
+// Which way nn takes when it has scratch, by the times of all three over four
+// scenes in the reference's point order and in no order (us: scan / caller's
+// tree, lowest to highest / sorted):
+//   64 points x 16,384 queries          24 /   7      /  55
+//   1,000     x 4,096                   10 /  14-23   /  46
+//   1,000     x 65,536                  91 /  94-132  / 112
+//   1,000     x 200,000                266 / 245-366  / 232
+//   4,000     x 2,048                   14 /  10-14   /  57
+//   4,000     x 65,536                 180 /  71-97   / 146
+//   8,192     x 16,384                 103 /  88-181  / 104
+//   16,384    x 4,096                   56 /  59-146  /  81
+//   100,000   x 1,024                   83 /  27-102  / 105
+//   100,000   x 8,192                  557 /  43-303  / 133
+//   200,003   x 8,192                    - /  47-109  / 151
+//   300,000   x 1,024                  231 / 140-2705 / 186
+//   1,000,000 x 256                    189 / 211-1180 / 283
+//   1,000,000 x 65,536                   - / 1858-5882 / 532
+//   2,000,000 x 256                    349 / 178-1294 / 314
+// The scan costs 0.7 ps per pair (all of 2,048 points for every block), the sorts
+// and boxes 30 to 300 us.  The tree's boxes are the caller's order: up to 4,096
+// points two levels of them bound any order's cost; past that it is up to four
+// times as fast as the sorted search on good orders and 45 times as slow on
+// bad ones (100,000 points in no order x 4,096: 5.0 ms against 0.11), so it is left.
+NNRoute nn_route(uint32_t num_points, uint32_t num_queries) {
+    if (num_points <= 64) return NNRoute::kTree; // one group of points
+    if (num_points <= 2048) return num_queries <= 65536 ? NNRoute::kScan : NNRoute::kSorted;
+    if (num_points <= 4096) return num_queries <= 2048 ? NNRoute::kScan : NNRoute::kTree;
+    const uint64_t pairs = (uint64_t)num_points * num_queries;
+    return pairs <= (1ull << 27) + std::min<uint64_t>(256ull * num_points, 1ull << 28)
+               ? NNRoute::kScan
+               : NNRoute::kSorted;
 }
 
 size_t nn_scratch_bytes(uint32_t num_points, uint32_t num_queries) {
-    if (nn_scans(num_points, num_queries)) return align256(8ull * std::max(num_queries, 1u));
-    return layout_of(num_points, num_queries).bytes;
+    switch (nn_route(num_points, num_queries)) {
+    case NNRoute::kScan: return align256(8ull * std::max(num_queries, 1u));
+    case NNRoute::kTree: return 0;
+    default: return layout_of(num_points, num_queries).bytes;
+    }
 }
 
 hipError_t launch_nn_sorted(const float *points, const float *tree, const float *queries,

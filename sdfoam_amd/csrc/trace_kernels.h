@@ -370,9 +370,11 @@ StartLayout start_layout(uint32_t num_rays);
 hipError_t launch_start_points(const float *rays, uint32_t num_rays, const float *points,
                                uint32_t num_points, const float *tree, uint32_t *start,
                                void *scratch, hipStream_t stream);
-// nn with scratch (nn_scratch_bytes): a scan of every point for few pairs
-// (nn_scans), else a search over sorted points (nn_sorted.hip).
-bool nn_scans(uint32_t num_points, uint32_t num_queries);
+// nn with scratch (nn_scratch_bytes): a scan of every point for few pairs, the
+// search over the caller's tree, or one over sorted points (nn_sorted.hip).
+enum class NNRoute { kScan, kTree, kSorted };
+NNRoute nn_route(uint32_t num_points, uint32_t num_queries);
+// (0 for the tree, and where the sorts could not be sized)
 size_t nn_scratch_bytes(uint32_t num_points, uint32_t num_queries);
 hipError_t launch_nn_brute(const float *points, const float *queries, uint32_t num_points,
                            uint32_t num_queries, uint32_t *indices, uint64_t *best,

@@ -1,6 +1,5 @@
-"""nn's two ways with scratch (a scan of every point, a search over points
-sorted for the call) at the edges of their groups and of the rule between
-them, against the host's exact nearest neighbour; queries with infinities and
+"""nn's ways with scratch (a scan of every point, the search over the tree, a
+search over points sorted for the call) at the edges of their groups, against the host's exact nearest neighbour; queries with infinities and
 NaN against the tree search."""
 
 import numpy as np
@@ -24,22 +23,27 @@ def _threads():
     return min(16, os.cpu_count() or 1)
 
 
-def _scans(n, m):
-    return n * m <= (1 << 27) + 256 * n
+def _way(n, m):
+    """The way the library takes, by the scratch it asks for."""
+    from sdfoam_amd import _lib
+
+    need = int(_lib.lib().sdf_nn_scratch_bytes(n, m))
+    return "tree" if need == 0 else "scan" if need == -(-8 * m // 256) * 256 else "sorted"
 
 
 # groups of 64 points: 4,096 is the most with one level of boxes, 262,144 with two
-@pytest.mark.parametrize("n,m,scans", [
-    (32, 1, True), (33, 257, True), (2048, 300, True), (2049, 256, True), (300_001, 65, True),
-    (4096, 33_025, False), (4097, 33_017, False), (262_144, 769, False), (262_145, 901, False),
+@pytest.mark.parametrize("n,m,way", [
+    (32, 1, "tree"), (33, 257, "tree"), (2048, 300, "scan"), (2049, 256, "scan"),
+    (300_001, 65, "scan"), (1500, 66_000, "sorted"), (4096, 33_025, "tree"),
+    (4097, 33_017, "sorted"), (262_144, 769, "sorted"), (262_145, 901, "sorted"),
 ])
-def test_nn_paths(torch_dev, oracle_lib, n, m, scans):
+def test_nn_paths(torch_dev, oracle_lib, n, m, way):
     import torch
 
     import sdfoam_amd
     from sdfoam_amd import _lib, scenes
 
-    assert _scans(n, m) == scans
+    assert _way(n, m) == way
     rng = np.random.default_rng(n + m)
     pts = rng.normal(size=(n, 3)).astype(np.float32)
     pts[n // 2] = pts[n // 3]  # a tie: the smaller index wins

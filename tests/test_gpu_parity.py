@@ -807,11 +807,10 @@ def test_aabb_tree_and_nn_exact(torch_dev, oracle_lib):
 
 @pytest.mark.parametrize("n", [32, 33, 64, 65, 129, 4096, 4097, 70_000, 300_000])
 def test_nn_tree_depths(torch_dev, oracle_lib, n):
-    """nn over trees of every shape the search distinguishes: one group of
-    points (n <= 64), the depth-6 boxes over points (n <= 4096), the depth-6
-    and depth-12 boxes held in LDS over points, and boxes below depth 12 read
-    from the tree (n > 262,144).  Duplicated points make ties, which go to
-    the smaller index; the host's exact nearest neighbour is the reference."""
+    """nn at point counts on both sides of the tree's levels (test_gpu_nn_routes
+    runs the search over the tree itself at them).  Duplicated points make ties,
+    which go to the smaller index; the host's exact nearest neighbour is the
+    reference."""
     import torch
 
     import sdfoam_amd
