@@ -12,9 +12,11 @@ namespace {
 // outputs.  CT: the walk reads a cell table and a padded copy of the caller's
 // offset table that names each face's neighbour, made for the frame
 // (scene_prep_kernel); else the caller's arrays, its unpadded table with
-// guarded loads. 
+// guarded loads.
 template <int L, bool NEUS, typename AT, int G, bool CT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT && G == 1 ? 6 : 1))) void render_kernel(RenderArgs a) {
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(CT && G == 1 ? 6 : 1))) void
+render_kernel(RenderArgs a) {
     static_assert(G == 1 || CT, "lanes share a pixel over the cell table only");
     constexpr uint32_t RB = CT ? cell_record_bytes(L, sizeof(AT)) : 0u;
     constexpr int nsh = (L + 1) * (L + 1);
@@ -159,6 +161,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT && G 
 
 } // namespace
 
+// Lanes per pixel: more where few pixels leave the chip idle.  ms with 1, 2, 4, 8
+// and 16 lanes (walk and tables; in brackets over the caller's arrays), fp32, SH degree 3:
+//   4,096 / 300k points  1.13  0.70  0.43  0.33  0.30  (1.11)
+//   77k / 100k           0.94  0.62  0.42  0.40  0.48  (0.91)
+//   307k / 300k          1.33  1.40  1.08              (1.29)
+//   481k / 1M            3.35  2.97  2.49              (3.40)
+//   750k / 1M            4.25  3.93  3.45              (4.36), another scene 3.93 4.74 4.68 (4.50)
+//   1.09M / 1M           4.60  4.77  4.57              (4.92), another scene 5.16 6.32 6.36 (5.53)
+//   250k / 30k           0.76  0.61  0.48              (0.81)
+static int render_lanes(uint32_t pixels, uint32_t num_points) {
+    if (pixels < 2ull * num_points) {
+        if (pixels <= 16384u) return 16;
+        if (pixels <= 49152u) return 8;
+        if (pixels <= 400000u) return 4;
+        return pixels <= 800000u ? 2 : 1;
+    }
+    if (pixels <= 8192u) return 8;
+    if (pixels <= 65536u) return 4;
+    return pixels <= 163840u ? 2 : 1;
+}
+
 template <int L, typename AT, int G, bool CT>
 static hipError_t launch_render_G(const RenderArgs &a, bool neus, hipStream_t stream) {
     const dim3 grid(grid_blocks_for_tiles(a.num_tiles) * G);
@@ -173,7 +196,7 @@ static hipError_t launch_render_G(const RenderArgs &a, bool neus, hipStream_t st
 template <int L, typename AT>
 static hipError_t launch_render_L(const RenderArgs &a, bool neus, hipStream_t stream) {
     if (!a.scene.cells) return launch_render_G<L, AT, 1, false>(a, neus, stream);
-    switch (forward_lanes(a.width * a.height, a.scene.num_points, false)) {
+    switch (render_lanes(a.width * a.height, a.scene.num_points)) {
     case 16: return launch_render_G<L, AT, 16, true>(a, neus, stream);
     case 8: return launch_render_G<L, AT, 8, true>(a, neus, stream);
     case 4: return launch_render_G<L, AT, 4, true>(a, neus, stream);

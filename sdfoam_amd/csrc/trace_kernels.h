@@ -261,9 +261,6 @@ hipError_t launch_forward(int L, const FwdArgs &a, bool neus, bool stats, bool h
 hipError_t launch_scene_prep(int L, bool half, const SceneView &sc, uint32_t *cells, uint2 *diff,
                              void *contribution, float *alpha, const uint2 *given,
                              hipStream_t stream);
-// Lanes per ray (1 to 16) of a walk over the cell table; `ordered`: rays in an
-// explicit launch order.
-int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered);
 // Floats per cell row of the backward's gradient accumulator: the next
 // power of two >= D + 4 (attribute row, position, point error), at least 8,
 // so that a row spans the fewest 64-byte segments.

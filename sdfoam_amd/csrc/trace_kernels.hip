@@ -186,9 +186,11 @@ __device__ __forceinline__ void contrib_flush(ContribTable<kContribSlots> &ct,
 constexpr int kForwardWaves = 6;
 
 // CT: walk over the cell table (a.scene.cells) and read attribute rows from it.
-template <int L, bool NEUS, bool STATS, typename AT, bool CT = false>
+// HALF: the face scan's half-batch loads (walk_advance), for rays in an
+// explicit launch order (incoherent batches such as random training pixels).
+template <int L, bool NEUS, bool STATS, typename AT, bool CT = false, bool HALF = false>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(CT && !STATS ? kForwardWaves : 1))) void
+__attribute__((amdgpu_waves_per_eu(CT && !HALF && !STATS ? kForwardWaves : 1))) void
 forward_kernel(FwdArgs a) {
     constexpr uint32_t RB = CT ? cell_record_bytes(L, sizeof(AT)) : 0u;
     constexpr int nsh = (L + 1) * (L + 1);
@@ -242,14 +244,14 @@ forward_kernel(FwdArgs a) {
         uint2 entry = make_uint2(kWalkUnrecorded, 0u);
         if (ws.alive) {
             if constexpr (NEUS || STATS) {
-                walk_advance<true, STATS, false, false, RB>(a.scene, ray, max_steps, ws, si, wc);
+                walk_advance<true, STATS, false, false, RB, HALF>(a.scene, ray, max_steps, ws, si, wc);
                 entry = make_uint2(si.found ? si.next : kNoIndex,
                                    __builtin_bit_cast(uint32_t, si.t1));
             } else {
                 // the density backward walks in the unsafe mode: a step is
                 // recorded while that walk takes the same exit; from the first
                 // step where it would not, the backward scans for itself
-                walk_advance<true, false, false, true, RB>(a.scene, ray, max_steps, ws, si, wc);
+                walk_advance<true, false, false, true, RB, HALF>(a.scene, ray, max_steps, ws, si, wc);
                 if (si.agrees)
                     entry = make_uint2(si.found ? si.next : kNoIndex,
                                        __builtin_bit_cast(uint32_t, si.t1));
@@ -903,8 +905,8 @@ __device__ __forceinline__ void publish_step(WaveTables<L, PE> &tb, StepEntries 
 // the rows).  They are sums of one sign, and a cell that all rays cross gets one
 // term per wavefront: with fewer rays per wavefront there are more of them to
 // round, 1.2e-6 against 0.7e-6 of the sums at 400x400 rays in fp32.
-// start_rows (ACC): the rows of the cells start_cells (in LDS) go there instead
-// (this block's copy of row 0), or NULL.
+// start_rows (ACC, G > 1): the rows of the cells start_cells (in LDS) go there
+// instead (this block's copy of row 0).
 // ALSO_LAST: the last channel is an SH component too (sdf_channel < 3 nsh).
 template <int L, bool PE, typename AT, bool ACC, bool ALSO_LAST, int G>
 __device__ __forceinline__ void grouped_pass_impl(StepEntries &e, const OwnerLane &ow,
@@ -1585,32 +1587,49 @@ static inline dim3 grid_for(uint64_t n) { return dim3((unsigned)((n + kBlock - 1
 // and a walk's time is its latency: more lanes shorten it.  More rays fill it,
 // and the work that the lanes of a ray repeat costs more than it gives; the
 // sooner, the more rays there are per cell (their wavefronts then share cells,
-// and end together).  The lines are where the two sides met over six scenes of
-// 4k to 3M points (ms, forward / backward):
-//   rays / points      1 lane       2            4            8            16
-//   6.7k / 300k      2.08/2.30     -/1.38     1.04/0.91    0.84/0.69    0.82/0.58
-//   20k batch / 300k 1.63/1.30     -/0.87     0.85/0.73    0.76/0.68    1.00/0.79
-//   65k batch / 200k 1.89/2.27  1.36/1.96     1.08/1.72    1.39/1.91    2.04/2.28
-//   307k / 1M        4.26/4.07  2.89/2.67     2.79/2.63    3.36/3.52    5.53/5.86
-//   750k / 1M        4.76/4.74  4.47/4.02     4.75/4.80
-//   1M batch / 2M    18.4/22.2  17.5/19.2     17.1/20.3
-//   1.9M / 1M        7.18/7.50  9.15/7.09     10.6/10.6
-//   32k / 4k         0.34/0.21  0.26/0.15     0.24/0.14    0.28/0.16    0.34/0.22
-//   90k / 10k        0.45/0.31  0.39/0.28     0.41/0.33    0.50/0.49    0.74/0.79
-//   202k / 30k       0.66/0.58  0.75/0.59     0.77/0.75    1.07/1.23    1.84/2.13
-//   900k / 30k       1.14/1.40  1.44/1.54     1.84/2.41
-// (two lanes shorten the backward even where the chip is full: 32 rays over six
-// trips meet fewer distinct cells than 64 rays over three).
-int forward_lanes(uint32_t num_rays, uint32_t num_points, bool ordered) {
+// and end together).  The lines are where the sides met over scenes of 4k to 3M
+// points ("object" / "blobs", fp32 unless it says fp16, SH degree 3), ms:
+//   image rays / points   forward: 1        2          4          8     backward: 1      2          4          8          16
+//   4.1k / 4.1k           0.41/0.30  0.24/0.18  0.17/0.13  0.14/0.11  0.34/0.32  0.24/0.21  0.17/0.15  0.14/0.12  0.13/0.11
+//   19k / 100k            0.96/0.92  0.57/0.52  0.41/0.39  0.32/0.32  1.02/1.22  0.79/0.79  0.55/0.52  0.43/0.41  0.39/0.40
+//   160k / 100k           0.99/0.87  0.79/0.76  0.63/0.65             1.33/1.00  0.86/0.72  0.78/0.79
+//   307k / 300k           1.52/1.47  1.51/1.58  1.34/1.59             2.04/1.70  1.61/1.40  1.62/1.91
+//    fp16                 1.45/1.38  1.33/1.35  1.38/1.66
+//   481k / 300k           1.75/1.82  1.93/2.32  1.79/2.41             2.34/1.91  1.93/1.96  2.12/2.85
+//   481k / 1M             3.49/3.58  3.32/3.84  3.03/3.93             3.89/3.47  3.21/3.09  3.31/4.30
+//   750k / 1M             4.09/4.22  4.38/5.57  4.27/5.76             4.79/4.28  4.00/4.40  4.51/6.32
+//   1.09M / 1M            4.86/5.11  5.67/7.69  5.75/7.98             4.95/4.93  4.59/5.98  6.06/8.81
+//   1.09M / 3M            8.14/8.76  8.37/11.5  8.49/11.9             8.93/8.72  7.32/9.28  8.83/13.0
+//   1.9M / 1M             6.44/7.99  9.70/13.0  9.99/13.7             6.53/7.70  7.08/9.97  10.7/15.2
+//   8.7M / 3M             62.9       95.3                             62.0       70.6
+//   250k / 30k            0.78/0.69  0.63/0.60  0.55/0.62             0.84/0.61  0.63/0.59  0.68/0.83
+//   random rays / points
+//   65k / 200k            1.13/1.42  0.75/0.95  0.55/0.71  0.79/0.96  1.24/1.74  1.04/1.42  0.90/1.17  1.00/1.33
+//   65k / 30k             0.65/0.67  0.40/0.45  0.31/0.35  0.43/0.48  0.66/0.86  0.53/0.71  0.45/0.55  0.57/0.66
+//   131k / 30k            0.69/0.74  0.61/0.67  0.54/0.60             0.81/0.98  0.66/0.83  0.74/0.87
+//   524k / 300k           2.88/3.97  2.99/3.74  2.77/3.57             4.56/5.56  3.88/4.83  3.64/4.81
+//    fp16, half loads     2.58/3.22  2.51/3.18  2.90/3.76
+//   1M / 1M               8.07/11.7  8.27/10.9  7.85/10.5             11.8/16.0  9.82/13.4  10.4/14.4
+//    fp16, half loads     6.65/8.74  6.94/9.31  7.99/10.6
+//   1M / 100k             2.66/3.30  3.54/4.27  3.43/4.27             3.51/4.62  3.37/4.19  4.21/5.26
+//   1M / 30k              1.71/1.93  2.32/2.71  2.29/2.75             2.04/2.40  2.12/2.52  2.78/3.41
+static int forward_lanes(const FwdArgs &a, bool half) {
+    const uint32_t num_rays = a.num_rays, num_points = a.scene.num_points;
+    const bool ordered = a.order != nullptr;
     if (num_rays < 2ull * num_points) {
         if (num_rays <= 16384u) return 16;
         if (num_rays <= 49152u) return 8;
-        if (ordered || num_rays <= 400000u) return 4;
-        return num_rays <= 800000u ? 2 : 1;
+        if (half) {
+            if (num_rays <= (ordered ? 98304u : 245760u)) return 4;
+            if (num_rays <= (ordered ? 614400u : 400000u)) return 2;
+            if (ordered) return 1;
+        } else if (ordered || num_rays <= 400000u) {
+            return 4;
+        }
+        return num_rays <= 800000u && 2ull * num_rays <= num_points ? 2 : 1;
     }
     if (num_rays <= 8192u) return 8;
     if (num_rays <= 65536u) return 4;
-    if (ordered) return num_rays < 16ull * num_points ? 2 : 1;
     return num_rays <= 163840u ? 2 : 1;
 }
 
@@ -1646,12 +1665,26 @@ static hipError_t launch_forward_L(const FwdArgs &a, bool neus, bool stats, hipS
     const bool ct = a.scene.cells != nullptr;
     // (fp16 sums keep their roundings: each atomic of theirs rounds to 11 bits)
     if (ct && !stats && !(sizeof(AT) == 2 && a.contribution)) {
-        switch (forward_lanes(a.num_rays, a.scene.num_points, a.order != nullptr)) {
+        switch (forward_lanes(a, sizeof(AT) == 2)) {
         case 16: return launch_forward_split<L, AT, 16>(a, neus, stream);
         case 8: return launch_forward_split<L, AT, 8>(a, neus, stream);
         case 4: return launch_forward_split<L, AT, 4>(a, neus, stream);
         case 2: return launch_forward_split<L, AT, 2>(a, neus, stream);
         default: break;
+        }
+    }
+    if constexpr (sizeof(AT) == 2) {
+        // half-batch face loads: with contribution 14.1 against 16.7 ms for 1M sorted
+        // rays over 2M points; many rays per cell share them and pay for the branch
+        // (1M over 30k points 1.76 against 1.66)
+        if (ct && !stats && a.order && a.num_rays < 8ull * a.scene.num_points) {
+            if (neus)
+                hipLaunchKernelGGL((forward_kernel<L, true, false, AT, true, true>), grid,
+                                   dim3(kBlock), 0, stream, a);
+            else
+                hipLaunchKernelGGL((forward_kernel<L, false, false, AT, true, true>), grid,
+                                   dim3(kBlock), 0, stream, a);
+            return hipGetLastError();
         }
     }
     if (neus) {
