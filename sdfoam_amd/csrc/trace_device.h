@@ -146,9 +146,12 @@ __device__ __forceinline__ uint32_t block_tile() {
 
 // Tile runs of the forward and the inference render (measured on a
 // 1600x1200 camera: the forward is about 13% faster than with one run per
-// XCD, the backward about 2% slower, so it keeps one run per XCD).
+// XCD) and of the backward with one lane per ray.  With one run per XCD the
+// backward's time was that of the XCD with the most work: 1600x1200 rays over 1M
+// points of eleven scenes took 6.5-11.2 ms, 6.3-8.6 in runs of four tiles (8 cameras
+// of 1,089,480 rays over 3M points 62.7 -> 61.9 ms; runs of 1 to 128 within 5% of it).
 constexpr uint32_t kForwardChunk = 128;
-constexpr uint32_t kBackwardChunk = 0;
+constexpr uint32_t kBackwardChunk = 4;
 
 // The ray this lane traces: with `order` (a permutation of the rays, see
 // order_kernels.hip) lane i of the launch takes ray order[i]; entries out of

@@ -1083,11 +1083,14 @@ __device__ __forceinline__ BackwardLane backward_lane(const BwdArgs &a) {
     BackwardLane b;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     if constexpr (G == 1) {
-        b.ray = ray_for_lane<kBackwardChunk>(a.num_rays, a.settings.ray_image_width, a.num_tiles,
-                                             b.valid, a.order);
-        b.row = block_tile<kBackwardChunk>() * (kBlock / 64) + wave;
+        // (sorted and random rays cost about the same everywhere: one run per XCD
+        // keeps more of a cell's rays on one)
+        const bool image = a.settings.ray_image_width != 0 && !a.order;
+        b.row = (image ? block_tile<kBackwardChunk>() : block_tile<0>()) * (kBlock / 64) + wave;
         b.pos = lane;
         b.sub = 0;
+        b.ray = ray_at(b.row, lane, a.num_rays, a.settings.ray_image_width, a.num_tiles, b.valid,
+                       a.order);
     } else {
         // wavefront `part` of the G that share a row of 64 rays
         const uint32_t wv = split_wave<G>(blockIdx.x) + wave;
@@ -1638,14 +1641,17 @@ static int backward_lanes(const BwdArgs &a) {
     // without the fp64 sums a cell that all rays cross would take more
     // rounded terms from more lanes per ray
     if (!a.start_sums || (a.point_error && !a.error_sums)) return 1;
+    const bool image = a.settings.ray_image_width != 0 && !a.order;
     if (num_rays < 2ull * num_points) {
         if (num_rays <= 16384u) return 16;
         if (num_rays <= 49152u) return 8;
-        return num_rays <= 330000u ? 4 : 2;
+        if (num_rays <= (image ? 245760u : 330000u)) return 4;
+        if (!image || num_rays <= 600000u) return 2;
+        return num_rays <= 1300000u && num_rays <= num_points ? 2 : 1;
     }
     if (num_rays <= 8192u) return 8;
-    if (num_rays <= 40960u) return 4;
-    return num_rays < 16ull * num_points ? 2 : 1;
+    if (num_rays <= (image ? 40960u : 81920u)) return 4;
+    return num_rays < 16ull * num_points && (!image || num_rays <= 600000u) ? 2 : 1;
 }
 
 template <int L, typename AT, int G>

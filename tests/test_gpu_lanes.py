@@ -1,13 +1,15 @@
 """The fp16 forward over the cell table, at every number of lanes per ray and with
 the half-batch face loads of sorted rays, against the one-lane forward over the
 caller's arrays (cell_table=False): every per-ray output and the walk record bit for
-bit, contributions within the bound of their roundings."""
+bit, contributions within the bound of their roundings; and the backward of either
+dtype where the number of its lanes changes, against the oracle."""
 
 import numpy as np
 import pytest
 
+from conftest import scene
 from test_gpu_fp16 import gamma_h, half_scene
-from test_gpu_parity import gpu_scene, record_rows, torch_dev  # noqa: F401
+from test_gpu_parity import _backward_both, _check_backward, gpu_scene, record_rows, torch_dev  # noqa: F401
 from test_gpu_split import cut
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +59,13 @@ def test_fp16_forward_same_bits(torch_dev, monkeypatch, cfg, shape, mode, contri
         ca, cb = (o["contribution"].double().cpu().numpy().ravel() for o in (a, b))
         # the same weights in two orders, every fp16 addition rounded
         assert (np.abs(ca - cb) <= 2 * gamma_h(w.num_rays) * np.abs(ca) + 1e-5).all()
+
+
+# one lane at a full chip (over 600,000 image rays, 81,920 and 163,840 otherwise); four and two
+# lanes on both sides of their lines
+@pytest.mark.parametrize("cfg,shape", [(1, (90, 911)), (1, (81_920,)), (1, (81_921,)),
+                                       (1, (256, 257)), (2, (448, 440)), (2, (501, 1201))])
+def test_backward_lines(torch_dev, oracle_lib, cfg, shape):
+    w = cut(scene(cfg), shape)
+    bwd, st, ref = _backward_both(w, torch_dev, oracle_lib, "sdfoam", ray_error=True, walk=True)
+    _check_backward(bwd, st, ref, w)
