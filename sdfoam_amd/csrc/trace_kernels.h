@@ -165,8 +165,9 @@ struct FwdArgs {
 // sums of the same terms, over 160 traces (4k to 400k points, 6k to 1.7M rays,
 // geometric means, one lane per ray with fp32 sums = 1): more lanes with fp32
 // sums 1.18 (attributes), 1.12 (positions) and 2.0 (sharpness), with these 1.00,
-// 0.94 and below 0.01.  They cost the backward 0.28 of 19.0 ms (1M random rays, 2M
-// points) and, for 64x64 rays, 6 of 91 us.  Every row is there kStartCopies
+// 0.94 and below 0.01 (images 1.10 +- 0.05 and 1.02 +- 0.09, batches 0.90 +- 0.06
+// and 0.87 +- 0.07).  The test per sum costs the backward 0.28 of 19.0 ms (1M random rays,
+// 2M points), 2% at 65k rays and, for 64x64 rays, 6 of 91 us.  Every row is there kStartCopies
 // times (blocks take turns): one copy alone took 3% of a 1600x1200 backward
 // waiting for atomics.  Zeroed but for `cells`.
 constexpr uint32_t kStartRows = 64, kStartCopies = 8;

@@ -138,6 +138,70 @@ def test_grad_accum_sizes_and_errors():
         assert rc == 1 and msg in L.sdf_last_error()
 
 
+def test_grad_sums_sizes():
+    from sdfoam_amd import _lib
+
+    L = _lib.lib()
+    # 8 bytes per point (a multiple of 16), then 64 cell numbers, the sharpness (16
+    # bytes) and 8 copies of 64 rows of doubles
+    assert [L.sdf_grad_sums_bytes(d, 11) for d in range(4)] == [
+        96 + 256 + 16 + 8 * 64 * 8 * s for s in (8, 32, 32, 64)]
+    assert L.sdf_grad_sums_bytes(4, 10) == 0 and L.sdf_grad_sums_bytes(-1, 10) == 0
+
+
+def test_output_flags():
+    """SDF_OUTPUTS_FRESH needs what writes the outputs; FINITE needs FRESH."""
+    from sdfoam_amd import _lib
+
+    L = _lib.lib()
+    s = _settings()
+    buf = (C.c_uint64 * 1024)()
+    p = C.cast(buf, C.c_void_p)
+    nb = L.sdf_trace_scratch_bytes(10, 4)
+    aligned = (C.cast(buf, C.c_void_p).value + 255) & ~255
+
+    def forward(plan):
+        return L.sdf_trace_forward_planned(C.byref(plan), 3, C.byref(s), 10, p, p, 4, p, p, 1, p,
+                                           p, 0, None, p, None, None, p, None, p, p, p, nb, None)
+
+    def backward(plan, rays=1):
+        return L.sdf_trace_backward_planned(C.byref(plan), 3, C.byref(s), 10, p, p, 4, p, p, rays,
+                                            p, p, 0, None, None, p, p, None, None, p, p, None, p,
+                                            None, p, nb, None)
+
+    fresh = _lib.TracePlanDesc()
+    fresh.outputs = _lib.SDF_OUTPUTS_FRESH
+    assert forward(fresh) == 1 and b"needs a cell table" in L.sdf_last_error()
+    assert backward(fresh) == 1 and b"rays and a gradient accumulator" in L.sdf_last_error()
+    fresh.grad_accum, fresh.grad_accum_bytes = aligned, 2560
+    assert backward(fresh, rays=0) == 1 and b"rays and a gradient accumulator" in L.sdf_last_error()
+    finite = _lib.TracePlanDesc()
+    finite.outputs = _lib.SDF_OUTPUTS_FINITE
+    finite.grad_accum, finite.grad_accum_bytes = aligned, 2560
+    assert backward(finite) == 1 and b"needs SDF_OUTPUTS_FRESH" in L.sdf_last_error()
+
+
+def test_nn_ways_and_errors():
+    """The scratch of nn's ways that need no sort, and its checks."""
+    from sdfoam_amd import _lib
+
+    L = _lib.lib()
+    for n, m, need in ((31, 5, 0), (32, 5, 0), (64, 9999, 0), (65, 0, 256), (65, 1, 256),
+                       (65, 33, 512), (2048, 65_536, 524_288), (2049, 2049, 0), (4096, 9, 256),
+                       (4096, 2049, 0), (4097, 33_016, 264_192), (1_000_000, 390, 3328)):
+        assert L.sdf_nn_scratch_bytes(n, m) == need, (n, m)
+    buf = (C.c_uint64 * 64)()
+    p = C.cast(buf, C.c_void_p)
+    aligned = (C.cast(buf, C.c_void_p).value + 255) & ~255
+    assert L.sdf_nn_planned(p, p, p, 31, 1, p, None, 0, None) == 1
+    assert b"at least 32" in L.sdf_last_error()
+    assert L.sdf_nn_planned(p, p, p, 100, 1, p, None, 0, None) == 1
+    assert b"scratch must hold 256 bytes" in L.sdf_last_error()
+    assert L.sdf_nn_planned(p, p, p, 100, 1, p, aligned + 8, 256, None) == 1
+    assert b"256-byte aligned" in L.sdf_last_error()
+    assert L.sdf_nn_planned(p, p, None, 100, 0, None, None, 0, None) == 0
+
+
 def test_cell_table_sizes_and_errors():
     from sdfoam_amd import _lib
 
