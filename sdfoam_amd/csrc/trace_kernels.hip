@@ -1,7 +1,8 @@
 // Forward / backward kernels of the Voronoi-foam tracer for gfx950, and the
 // fp16 neighbour-offset prepass.
 //
-// One lane per ray, wave64, 256 lanes per block.  The walk is wave
+// One lane per ray (up to 16 neighbouring ones where rays are few: trace_split.h),
+// wave64, 256 lanes per block.  The walk is wave
 // synchronous: every trip of the kernel's loop advances each live lane by one
 // cell (the divergent part: face scan and the step's arithmetic), then the
 // whole wave reconverges and applies the step's scattered updates grouped by
@@ -380,9 +381,10 @@ forward_kernel(FwdArgs a) {
 // With few rays the chip is not full and a walk's time is its latency: one
 // lane per ray scans a cell's ~16 faces one after another, in batches that each
 // wait for their loads (216 us for 44 trips at 64x64 rays and 4,104 cells, 4.7 us
-// a trip; 85 us with 16 lanes per ray).  Here G neighbouring lanes share a ray: they scan the faces G at a time (consecutive lanes read
-// consecutive table entries), combine the exits by DPP, and carry the same
-// walk state; three of them form one colour channel each.  The exit face is
+// a trip; 85 us with 16 lanes per ray).  Here G neighbouring lanes share a ray:
+// they scan the faces G at a time (consecutive lanes read consecutive table
+// entries), combine the exits by DPP, and carry the same walk state; with four
+// lanes or more, three of them form one colour channel each.  The exit face is
 // the first minimum in row order as in walk_advance, every product and sum of
 // a step is the same one, so all outputs keep their bits.
 //
@@ -1740,8 +1742,9 @@ hipError_t launch_record_reset(const WalkRecordArgs &r, uint64_t table_words, hi
 // table's zero padding, as prefetch_diff_kernel does.  Record words past the
 // attribute row are left unwritten (nothing reads them).  The offset table
 // built with the cell table (from the points, or from a caller's table:
-// `given`) carries each entry's neighbour in its fourth half (`neighbour_delta`), so the walk over the cell table reads the exit
-// face's neighbour from the entry it already holds.  CELLS = false: the
+// `given`) carries each entry's neighbour in its fourth half
+// (`neighbour_delta`), so the walk over the cell table reads the exit face's
+// neighbour from the entry it already holds.  CELLS = false: the
 // offset table alone, as prefetch_adjacent_diff gives it (fourth half 0).
 template <int L, typename AT, bool CELLS = true>
 __global__ __launch_bounds__(kBlock) void scene_prep_kernel(const SceneView sc, uint32_t *cells,
